@@ -121,8 +121,7 @@ struct Slots {
   static constexpr int JS = EWT + N1;                 // Jacobian accumulation (copied to the matrix region)
   static constexpr int FY = JS + N1 * N1;             // species forcing (N1-1)
   static constexpr int TMP = FY + N1;                 // N1 scratch vector
-  static constexpr int ATOL = TMP + N1;               // N1
-  static constexpr int Y = ATOL + N1;                 // evaluation point of this trip
+  static constexpr int Y = TMP + N1;                  // evaluation point of this trip
   static constexpr int F = Y + N1;                    // right-hand side at Y
   static constexpr int TS = F + N1;                   // temperature re-solved at Y
   static constexpr int SING = TS + 1;                 // 0, or 1 + first zero-pivot column of the last LU
@@ -267,12 +266,17 @@ __device__ __forceinline__ void rhs(const double* __restrict__ y, const double t
   f[N] = (fH - hw * M::RU * T) / (rhocp * M::RU);
 }
 
-// analytic Jacobian of the right-hand side at (y, T) with T held fixed, into ws[JS].
-// Every entry is written once (no accumulation in memory); the T row's sum over a
-// column is formed as that column's entries are produced.
+// analytic Jacobian of the right-hand side at (y, T) with T held fixed, into js[JS] (the
+// forcing is read from the cell's own tile ws).  Every entry is written once (no
+// accumulation in memory); the T row's sum over a column is formed as that column's
+// entries are produced.
+// The tiles come by value: by reference their addresses are reloaded from the stack after
+// every store of an entry, which may alias them.
 template <class M>
-__device__ __noinline__ void jacobian(const double* __restrict__ y, const double T, const double fT, const WS& ws) {
+__device__ __noinline__ void jacobian(const double* __restrict__ y, const double T, const double fT, const WS ws,
+                                      const WS js) {
   constexpr int N = M::NS, N1 = M::N1;
+  auto at = [&](int i, int k) -> double& { return js[Slots<N1>::JS + i * N1 + k]; };
   using S = Slots<N1>;
   const double logT = log(T), invT = 1.0 / T;
   double C[N], g[N], hRT[N], cpR[N], wd[N], dwdT[N];
@@ -289,11 +293,11 @@ __device__ __noinline__ void jacobian(const double* __restrict__ y, const double
   double s = 0.0;
   M::jacobian(C, T, logT, invT, g, hRT, wd, dwdT,
               [&](int i, int k, double v) {
-                ws[S::JS + i * N1 + k] = v;
+                at(i, k) = v;
                 s += hRT[i] * M::imw(i) * v;
               },
               [&](int k) {
-                ws[S::JS + N * N1 + k] = (-M::RU * T * s - fT * M::RU * cpR[k] * M::imw(k)) / rhocp;
+                at(N, k) = (-M::RU * T * s - fT * M::RU * cpR[k] * M::imw(k)) / rhocp;
                 s = 0.0;
               });
   double dcp[N];
@@ -303,29 +307,42 @@ __device__ __noinline__ void jacobian(const double* __restrict__ y, const double
   for (int k = 0; k < N; ++k) {
     drhocp += y[k] * dcp[k] * M::imw(k);
     sTT += cpR[k] * (wd[k] + ws[S::FY + k] * M::imw(k)) + hRT[k] * T * dwdT[k];
-    ws[S::JS + k * N1 + N] = M::mw(k) * dwdT[k];
+    at(k, N) = M::mw(k) * dwdT[k];
   }
   drhocp *= M::RU;
-  ws[S::JS + N * N1 + N] = (-M::RU * sTT - fT * drhocp) / rhocp;
+  at(N, N) = (-M::RU * sTT - fT * drhocp) / rhocp;
+}
+template <class M>
+__device__ __forceinline__ void jacobian(const double* __restrict__ y, const double T, const double fT, const WS& ws) {
+  jacobian<M>(y, T, fT, ws, ws);
 }
 
 // ---------------------------------------------------------------------------
 // dense LU of M = I - gamma J (partial pivoting, whole-row interchanges) and solve
 // ---------------------------------------------------------------------------
-// Factors of I - gamma J in the matrix region: FP64 one per word, or FP32 contiguous
-// (element e at float index e of the region).
+// Factors of I - gamma J in the matrix region: FP64 one per word, or FP32 contiguous.
+// They are stored by columns: at(m, i, j) is element (i, j) of the factors, at(m, e) the
+// one at row-major position e.  The cooperative kernels hold one row per lane, so a load
+// or store of column j by a cell's lanes covers N1 consecutive words (two or three lines)
+// where rows would touch one line per lane (solves of drm19 128^3 by rows 49.8 ms, by
+// columns 43.7 ms; of the 53-species 64^3 box 60.5 and 52.0 ms; the factorisations the same).
 template <int N1, class Real>
 struct LUAcc;
 template <int N1>
 struct LUAcc<N1, double> {
-  static __device__ __forceinline__ double& at(const CM& m, int e) { return m[MatSlots<N1>::LU + e]; }
+  static __device__ __forceinline__ double& at(const CM& m, int i, int j) {
+    PELE_CHECK(i >= 0 && i < N1 && j >= 0 && j < N1, "FP64 factor", i * N1 + j, N1 * N1);
+    return m[MatSlots<N1>::LU + j * N1 + i];
+  }
+  static __device__ __forceinline__ double& at(const CM& m, int e) { return at(m, e / N1, e % N1); }
 };
 template <int N1>
 struct LUAcc<N1, float> {
-  static __device__ __forceinline__ float& at(const CM& m, int e) {
-    PELE_CHECK(e >= 0 && e < N1 * N1, "FP32 factor", e, N1 * N1);
-    return reinterpret_cast<float*>(&m[MatSlots<N1>::LU])[e];
+  static __device__ __forceinline__ float& at(const CM& m, int i, int j) {
+    PELE_CHECK(i >= 0 && i < N1 && j >= 0 && j < N1, "FP32 factor", i * N1 + j, N1 * N1);
+    return reinterpret_cast<float*>(&m[MatSlots<N1>::LU])[j * N1 + i];
   }
+  static __device__ __forceinline__ float& at(const CM& m, int e) { return at(m, e / N1, e % N1); }
 };
 
 // one lane factors its cell's M = I - gamma J (partial pivoting, arithmetic in Real);
@@ -338,16 +355,16 @@ __device__ __noinline__ int lu_factor(const CM& mat, const double gamma) {
   for (int i = 0; i < N1; ++i) {
     mat.perm(MS::PERM, i) = i;
 #pragma unroll
-    for (int j = 0; j < N1; ++j) A::at(mat, i * N1 + j) = (Real)((i == j ? 1.0 : 0.0) - gamma * mat[MS::JS + i * N1 + j]);
+    for (int j = 0; j < N1; ++j) A::at(mat, i, j) = (Real)((i == j ? 1.0 : 0.0) - gamma * mat[MS::JS + i * N1 + j]);
   }
   int sing = 0;
 #pragma unroll 1
   for (int k = 0; k < N1; ++k) {
     int p = k;
-    Real amax = fabs(A::at(mat, k * N1 + k));
+    Real amax = fabs(A::at(mat, k, k));
 #pragma unroll 1
     for (int i = k + 1; i < N1; ++i) {
-      const Real a = fabs(A::at(mat, i * N1 + k));
+      const Real a = fabs(A::at(mat, i, k));
       if (a > amax) { amax = a; p = i; }
     }
     if (amax == (Real)0) { if (!sing) sing = k + 1; continue; }
@@ -357,19 +374,19 @@ __device__ __noinline__ int lu_factor(const CM& mat, const double gamma) {
       mat.perm(MS::PERM, p) = t;
 #pragma unroll 1
       for (int j = 0; j < N1; ++j) {
-        const Real t2 = A::at(mat, k * N1 + j);
-        A::at(mat, k * N1 + j) = A::at(mat, p * N1 + j);
-        A::at(mat, p * N1 + j) = t2;
+        const Real t2 = A::at(mat, k, j);
+        A::at(mat, k, j) = A::at(mat, p, j);
+        A::at(mat, p, j) = t2;
       }
     }
-    const Real inv = (Real)1 / A::at(mat, k * N1 + k);
+    const Real inv = (Real)1 / A::at(mat, k, k);
 #pragma unroll 1
     for (int i = k + 1; i < N1; ++i) {
-      const Real lik = A::at(mat, i * N1 + k) * inv;
-      A::at(mat, i * N1 + k) = lik;
+      const Real lik = A::at(mat, i, k) * inv;
+      A::at(mat, i, k) = lik;
       if (lik != (Real)0) {
 #pragma unroll 1
-        for (int j = k + 1; j < N1; ++j) A::at(mat, i * N1 + j) -= lik * A::at(mat, k * N1 + j);
+        for (int j = k + 1; j < N1; ++j) A::at(mat, i, j) -= lik * A::at(mat, k, j);
       }
     }
   }
@@ -390,14 +407,14 @@ __device__ __forceinline__ void lu_solve(const CM& mat, const int src, const int
   for (int k = 0; k < N1; ++k) {
     const double xk = mat[dst + k];
 #pragma unroll 1
-    for (int i = k + 1; i < N1; ++i) mat[dst + i] -= (double)A::at(mat, i * N1 + k) * xk;
+    for (int i = k + 1; i < N1; ++i) mat[dst + i] -= (double)A::at(mat, i, k) * xk;
   }
 #pragma unroll 1
   for (int k = N1 - 1; k >= 0; --k) {
     double s = mat[dst + k];
 #pragma unroll 1
-    for (int j = k + 1; j < N1; ++j) s -= (double)A::at(mat, k * N1 + j) * mat[dst + j];
-    mat[dst + k] = s / (double)A::at(mat, k * N1 + k);
+    for (int j = k + 1; j < N1; ++j) s -= (double)A::at(mat, k, j) * mat[dst + j];
+    mat[dst + k] = s / (double)A::at(mat, k, k);
   }
 }
 
@@ -405,6 +422,10 @@ template <class M>
 struct Lane {
   static constexpr int N = M::NS, N1 = M::N1;
   using S = Slots<N1>;
+  // Loops over the components that touch the workspace, rolled: two iterations' loads in
+  // flight per wave suffice at three waves per SIMD, and unrolled whole the step kernel is
+  // 90 kB of code at 22 unknowns instead of 46 (93 against 90 ms on drm19 128^3).
+  static constexpr int PASS_UNROLL = 2;
   // -- persistent state: the words stored in the LANE slots between kernels (8-byte
   // members first, then 4-byte ones, then flags, so that no word is padding) --
   // history / step control
@@ -446,7 +467,6 @@ struct Lane {
   WS ws;
   IWS iws;
   CM mat;
-  const double* xs;   // this trip's Newton solution (matrix region, or its LDS copy)
   int qmax;
   double rtol;
   long mxstep;
@@ -459,103 +479,14 @@ struct Lane {
 
   __device__ __forceinline__ double& zn(int j, int i) const { return ws[S::ZN + j * N1 + i]; }
 
-  __device__ void ewtset() {
-    for (int i = 0; i < N1; ++i) ws[S::EWT + i] = 1.0 / (rtol * fabs(zn(0, i)) + ws[S::ATOL + i]);
-  }
-  // ewtset() and then the WRMS norm of zn0 with the new weights, in one pass
-  __device__ double ewtset_wrms_zn0() {
-    double s = 0.0;
-#pragma unroll 2
-    for (int i = 0; i < N1; ++i) {
-      const double z = zn(0, i);
-      const double e = 1.0 / (rtol * fabs(z) + ws[S::ATOL + i]);
-      ws[S::EWT + i] = e;
-      const double p = z * e;
-      s += p * p;
-    }
-    return sqrt(s / N1);
-  }
-  __device__ double wrms_ws(int slot) const {
-    double s = 0.0;
-#pragma unroll
-    for (int i = 0; i < N1; ++i) {
-      const double p = ws[slot + i] * ws[S::EWT + i];
-      s += p * p;
-    }
-    return sqrt(s / N1);
-  }
-  __device__ double wrms_reg(const double* v) const {
-    double s = 0.0;
-#pragma unroll
-    for (int i = 0; i < N1; ++i) {
-      const double p = v[i] * ws[S::EWT + i];
-      s += p * p;
-    }
-    return sqrt(s / N1);
+  __device__ __forceinline__ void ewtset(const ReactArgs& a) {
+#pragma unroll PASS_UNROLL
+    for (int i = 0; i < N1; ++i) ws[S::EWT + i] = 1.0 / (rtol * fabs(zn(0, i)) + a.atol[i]);
   }
 
-  // The Nordsieck updates below take each component's column zn(0..q, i) into
-  // registers once, apply the same operations in the same order as the column-at-a-
-  // time loops (so the results are identical), and store it once.
-  //
-  // start of an attempt: optionally rescale (zn(j) *= eta^j, h = hscale eta) and save
-  // y_n = zn0 in TMP, then predict (tn += h; zn(j-1) += zn(j) for k = 1..q, j = q..k),
-  // and clear acor
-  __device__ void rescale_predict(const bool do_rescale, const bool save_y) {
-    double fac[LMAX];
-    double factor = eta;
-    fac[0] = 1.0;
-#pragma unroll
-    for (int j = 1; j < LMAX; ++j) {
-      fac[j] = factor;
-      factor *= eta;
-    }
-    if (do_rescale) {
-      h = hscale * eta;
-      hscale = h;
-    }
-    tn += h;
-#pragma unroll 2
-    for (int i = 0; i < N1; ++i) {
-      double z[LMAX];
-#pragma unroll
-      for (int j = 0; j < LMAX; ++j) z[j] = (j <= q) ? zn(j, i) : 0.0;
-      if (save_y) ws[S::TMP + i] = z[0];
-      if (do_rescale) {
-#pragma unroll
-        for (int j = 1; j < LMAX; ++j)
-          if (j <= q) z[j] *= fac[j];
-      }
-#pragma unroll
-      for (int k = 1; k < LMAX; ++k)
-#pragma unroll
-        for (int j = LMAX - 1; j >= k; --j)
-          if (k <= q && j <= q) z[j - 1] += z[j];
-#pragma unroll
-      for (int j = 0; j < LMAX; ++j)
-        if (j < q || (j == q && do_rescale)) zn(j, i) = z[j];
-      ws[S::ACOR + i] = 0.0;
-    }
-  }
-  // undo the prediction: zn(j-1) -= zn(j) for k = 1..q, j = q..k
-  __device__ void restore() {
-    tn = saved_t;
-#pragma unroll 2
-    for (int i = 0; i < N1; ++i) {
-      double z[LMAX];
-#pragma unroll
-      for (int j = 0; j < LMAX; ++j) z[j] = (j <= q) ? zn(j, i) : 0.0;
-#pragma unroll
-      for (int k = 1; k < LMAX; ++k)
-#pragma unroll
-        for (int j = LMAX - 1; j >= k; --j)
-          if (k <= q && j <= q) z[j - 1] -= z[j];
-#pragma unroll
-      for (int j = 0; j < LMAX - 1; ++j)
-        if (j < q) zn(j, i) = z[j];
-    }
-  }
-  __device__ void increase_bdf() {
+  // the coefficients l (and the return value A1) that add a column to the Nordsieck array:
+  // zn(L) = A1 zn(qmax), the saved correction, and zn(j) += l[j] zn(L), j = 2..q
+  __device__ __forceinline__ double increase_coeffs() {
     for (int i = 0; i <= qmax; ++i) l[i] = 0.0;
     l[2] = 1.0;
     double alpha1 = 1.0, prod = 1.0, xiold = 1.0, alpha0 = -1.0, hsum = hscale;
@@ -570,14 +501,10 @@ struct Lane {
         xiold = xi;
       }
     }
-    const double A1 = (-alpha0 - alpha1) / prod;
-#pragma unroll
-    for (int i = 0; i < N1; ++i) zn(L, i) = A1 * zn(qmax, i);
-    for (int j = 2; j <= q; ++j)
-#pragma unroll
-      for (int i = 0; i < N1; ++i) zn(j, i) += l[j] * zn(L, i);
+    return (-alpha0 - alpha1) / prod;
   }
-  __device__ void decrease_bdf() {
+  // the coefficients l that drop column q: zn(j) -= l[j] zn(q), j = 2..q-1
+  __device__ __forceinline__ void decrease_coeffs() {
     for (int i = 0; i <= qmax; ++i) l[i] = 0.0;
     l[2] = 1.0;
     double hsum = 0.0;
@@ -586,15 +513,22 @@ struct Lane {
       const double xi = hsum / hscale;
       for (int i = j + 2; i >= 2; --i) l[i] = l[i] * xi + l[i - 1];
     }
+  }
+  __device__ void increase_bdf() {
+    const double A1 = increase_coeffs();
+#pragma unroll
+    for (int i = 0; i < N1; ++i) zn(L, i) = A1 * zn(qmax, i);
+    for (int j = 2; j <= q; ++j)
+#pragma unroll
+      for (int i = 0; i < N1; ++i) zn(j, i) += l[j] * zn(L, i);
+  }
+  __device__ void decrease_bdf() {
+    decrease_coeffs();
     for (int j = 2; j < q; ++j)
 #pragma unroll
       for (int i = 0; i < N1; ++i) zn(j, i) -= l[j] * zn(q, i);
   }
-  __device__ void adjust_order(int dq) {
-    if (q == 2 && dq != 1) return;
-    if (dq == 1) increase_bdf(); else decrease_bdf();
-  }
-  __device__ void set_coeffs() {
+  __device__ __forceinline__ void set_coeffs() {
     l[0] = l[1] = 1.0;
     double xi_inv = 1.0, xistar_inv = 1.0;
     for (int i = 2; i <= q; ++i) l[i] = 0.0;
@@ -641,140 +575,12 @@ struct Lane {
     gamrat = (nst > 0) ? gamma / gammap : 1.0;
   }
 
-  // start one attempt of the current step: predict, coefficients, Newton set-up
-  // (do_rescale: the step size changes by eta first)
-  __device__ void attempt(const bool do_rescale) {
-    // with the predictor, the state at tn (before the Nordsieck prediction) is the
-    // network's input
-    pred_state = use_pred ? 1 : 0;
-    rescale_predict(do_rescale, use_pred != 0);
-    set_coeffs();
-    convfail = (nflag == FIRST_CALL || nflag == PREV_ERR_FAIL) ? NO_FAILURES : FAIL_OTHER;
-    callSetup = (nflag == PREV_CONV_FAIL) || (nflag == PREV_ERR_FAIL) || (nst == 0) ||
-                (nst >= nstlp + MSBP) || (fabs(gamrat - 1.0) > DGMAX);
-    if (gmres) {   // no set-up function: nothing to refresh, the rate estimate restarts
-      callSetup = false;
-      crate = 1.0;
-    }
-    m = 0;
-    a1 = 0.0; a2 = 0.0; teval = tn;
-    phase = PH_NEWTON;
-  }
-  __device__ void finish(int st) {
+  __device__ __forceinline__ void finish(int st) {
     status = st;
     phase = PH_NEED_CELL;
   }
-  __device__ void loop_top() {
-    const double zn0_norm = (nst > 0) ? ewtset_wrms_zn0() : wrms_ws(S::ZN);
-    if (nstloc >= mxstep) { finish(ST_TOO_MUCH_WORK); return; }
-    const double tolsf = UROUND * zn0_norm;
-    if (tolsf > 1.0) { finish(ST_TOO_MUCH_ACC); return; }
-    saved_t = tn;
-    ncf = nef = 0;
-    nflag = FIRST_CALL;
-    const bool new_h = nst > 0 && hprime != h;
-    if (new_h && qprime != q) {
-      adjust_order(qprime - q);
-      q = qprime;
-      L = q + 1;
-      qwait = L;
-    }
-    attempt(new_h);
-  }
-  __device__ void begin_integration() {
-    hscale = h;
-    hprime = h;
-#pragma unroll
-    for (int i = 0; i < N1; ++i) zn(1, i) *= h;
-    nstloc = 0;
-    loop_top();
-  }
-  __device__ void hin_done() {
-    double h0 = H_BIAS * hnew;
-    if (h0 < hlb) h0 = hlb;
-    if (h0 > hub) h0 = hub;
-    h = h0;
-    begin_integration();
-  }
 
-  // the first right-hand side, f(0, y0), has been evaluated into zn1
-  __device__ void after_f0() {
-    const double tdist = tout;
-    const double tround = UROUND * tout;
-    if (tdist < 2.0 * tround) { finish(ST_TOO_CLOSE); return; }
-    hlb = HLB_FACTOR * tround;
-    double hub_inv = 0.0;
-#pragma unroll
-    for (int i = 0; i < N1; ++i) {
-      const double t1 = HUB_FACTOR * fabs(zn(0, i)) + ws[S::ATOL + i];
-      hub_inv = fmax(hub_inv, fabs(zn(1, i)) / t1);
-    }
-    hub = HUB_FACTOR * tdist;
-    if (hub * hub_inv > 1.0) hub = 1.0 / hub_inv;
-    hg = sqrt(hlb * hub);
-    if (hub < hlb) {
-      h = hg;
-      begin_integration();
-      return;
-    }
-    count1 = 1;
-    phase = PH_HIN;
-    a1 = hg; a2 = 0.0; teval = hg;
-  }
-  __device__ void after_hin(const double* f) {
-    double s = 0.0;
-#pragma unroll
-    for (int i = 0; i < N1; ++i) {
-      const double d = (f[i] - zn(1, i)) / hg * ws[S::EWT + i];
-      s += d * d;
-    }
-    const double yddnrm = sqrt(s / N1);
-    hnew = (yddnrm * hub * hub > 2.0) ? sqrt(2.0 / yddnrm) : sqrt(hg * hub);
-    if (count1 == HIN_ITERS) { hin_done(); return; }
-    const double hrat = hnew / hg;
-    if (hrat > 0.5 && hrat < 2.0) { hin_done(); return; }
-    if (count1 > 1 && hrat > 2.0) { hnew = hg; hin_done(); return; }
-    hg = hnew;
-    ++count1;
-    a1 = hg; a2 = 0.0; teval = hg;
-  }
-
-  __device__ void conv_failure() {
-    ++ncfn;
-    restore();
-    ++ncf;
-    etamax = 1.0;
-    if (ncf == MXNCF) { finish(ST_CONV_FAIL); return; }
-    eta = ETACF;
-    nflag = PREV_CONV_FAIL;
-    attempt(true);
-  }
-  __device__ void nls_fail() {
-    if (pred_state == 2) {
-      // the learned initial iterate did not converge: retry the same step from the
-      // Nordsieck prediction (the matrix set up in this attempt stays valid)
-      ++npredfb;
-      pred_state = 3;
-      callSetup = false;
-      m = 0;
-#pragma unroll
-      for (int i = 0; i < N1; ++i) ws[S::ACOR + i] = 0.0;
-      a1 = 0.0; a2 = 0.0; teval = tn;
-      return;
-    }
-    if (!jcur && !gmres) {
-      callSetup = true;
-      convfail = FAIL_BAD_J;
-      m = 0;
-#pragma unroll
-      for (int i = 0; i < N1; ++i) ws[S::ACOR + i] = 0.0;
-      a1 = 0.0; a2 = 0.0; teval = tn;
-      return;
-    }
-    conv_failure();
-  }
-
-  __device__ void set_eta() {
+  __device__ __forceinline__ void set_eta() {
     if (eta < THRESH) {
       eta = 1.0;
       hprime = h;
@@ -783,39 +589,38 @@ struct Lane {
       hprime = h * eta;
     }
   }
-  __device__ void prepare_next_step() {
+  // the step-size factor for an error test measure and its order's exponent
+  __device__ __forceinline__ static double eta_of(const double bias, const double d, const double k) {
+    return 1.0 / (pow(bias * d, 1.0 / k) + ADDON);
+  }
+  // The next step's size and order after a step of order q with etaq = eta_of(BIAS2, dsm,
+  // L).  sums(cquot, sq, sd) gives, for an order change (qwait = 0), the sums over the
+  // components of (zn(q) ewt)^2 and ((acor - cquot zn(qmax)) ewt)^2.  True when the order
+  // rises: zn(qmax) must then hold acor.
+  template <class Sums>
+  __device__ __forceinline__ bool choose_next(const double etaq, const Sums& sums) {
     if (etamax == 1.0) {
       qwait = max(qwait, 2);
       qprime = q;
       hprime = h;
       eta = 1.0;
-      return;
+      return false;
     }
-    const double etaq = 1.0 / (pow(BIAS2 * dsm, 1.0 / L) + ADDON);
     if (qwait != 0) {
       eta = etaq;
       qprime = q;
       set_eta();
-      return;
+      return false;
     }
     qwait = 2;
-    double etaqm1 = 0.0, etaqp1 = 0.0;
-    if (q > 1) {
-      const double ddn = wrms_ws(S::ZN + q * N1) * tq[1];
-      etaqm1 = 1.0 / (pow(BIAS1 * ddn, 1.0 / q) + ADDON);
-    }
-    if (q != qmax && saved_tq5 != 0.0) {
-      const double cquot = (tq[5] / saved_tq5) * pow(h / tau[2], (double)L);
-      double s = 0.0;
-#pragma unroll
-      for (int i = 0; i < N1; ++i) {
-        const double d = (ws[S::ACOR + i] - cquot * zn(qmax, i)) * ws[S::EWT + i];
-        s += d * d;
-      }
-      const double dup = sqrt(s / N1) * tq[3];
-      etaqp1 = 1.0 / (pow(BIAS3 * dup, 1.0 / (L + 1)) + ADDON);
-    }
+    const bool up = q != qmax && saved_tq5 != 0.0;
+    const double cquot = up ? (tq[5] / saved_tq5) * pow(h / tau[2], (double)L) : 0.0;
+    double sq = 0.0, sd = 0.0, etaqm1 = 0.0, etaqp1 = 0.0;
+    sums(cquot, sq, sd);
+    if (q > 1) etaqm1 = eta_of(BIAS1, sqrt(sq / N1) * tq[1], (double)q);
+    if (up) etaqp1 = eta_of(BIAS3, sqrt(sd / N1) * tq[3], (double)(L + 1));
     const double etam = fmax(etaqm1, fmax(etaq, etaqp1));
+    bool rise = false;
     if (etam < THRESH) {
       eta = 1.0;
       qprime = q;
@@ -828,122 +633,64 @@ struct Lane {
     } else {
       eta = etaqp1;
       qprime = q + 1;
-#pragma unroll
-      for (int i = 0; i < N1; ++i) zn(qmax, i) = ws[S::ACOR + i];
+      rise = true;
     }
     set_eta();
+    return rise;
   }
-
-  // Newton converged: error test, then complete the step or retry
-  __device__ bool after_converged() {   // returns true when tout has been reached
-    dsm = acnrm * tq[2];
-    if (!(dsm <= 1.0)) {   // a NaN norm fails the test, as in CVODE
-      ++nef;
-      ++netf;
-      nflag = PREV_ERR_FAIL;
-      restore();
-      if (nef == MXNEF) { finish(ST_ERR_FAIL); return false; }
-      etamax = 1.0;
-      if (nef <= MXNEF1) {
-        eta = 1.0 / (pow(BIAS2 * dsm, 1.0 / L) + ADDON);
-        eta = fmax(ETAMIN, eta);
-        if (nef >= SMALL_NEF) eta = fmin(eta, ETAMXF);
-        attempt(true);
-        return false;
+  // the same on a completed step's Nordsieck array and correction in the workspace
+  __device__ void prepare_next_step() {
+    const bool rise = choose_next(eta_of(BIAS2, dsm, (double)L), [&](const double cquot, double& sq, double& sd) {
+      for (int i = 0; i < N1; ++i) {
+        const double e = ws[S::EWT + i];
+        const double p = zn(q, i) * e;
+        sq += p * p;
+        const double d = (ws[S::ACOR + i] - cquot * zn(qmax, i)) * e;
+        sd += d * d;
       }
-      if (q > 1) {
-        eta = ETAMIN;
-        adjust_order(-1);
-        L = q;
-        --q;
-        qwait = L;
-        attempt(true);
-        return false;
-      }
-      eta = ETAMIN;
-      h *= eta;
-      hscale = h;
-      qwait = LONG_WAIT;
-      phase = PH_RESTART_F;
-      a1 = 0.0; a2 = 0.0; teval = tn;
-      return false;
-    }
-    // complete the step
-    ++nst;
-    for (int i = q; i >= 2; --i) tau[i] = tau[i - 1];
-    if (q == 1 && nst > 1) tau[2] = tau[1];
-    tau[1] = h;
-#pragma unroll 2
-    for (int i = 0; i < N1; ++i) {
-      const double ac = ws[S::ACOR + i];
-#pragma unroll
-      for (int j = 0; j < LMAX; ++j)
-        if (j <= q) zn(j, i) += l[j] * ac;
-    }
-    --qwait;
-    if (qwait == 1 && q != qmax) {
+    });
+    if (rise)
 #pragma unroll
       for (int i = 0; i < N1; ++i) zn(qmax, i) = ws[S::ACOR + i];
-      saved_tq5 = tq[5];
-    }
-    prepare_next_step();
-    etamax = (nst <= SMALL_NST) ? ETAMX2 : ETAMX3;
-    ++nstloc;
-    if ((tn - tout) * h >= 0.0) return true;
-    loop_top();
-    return false;
   }
 
-  __device__ bool needs_setup() const { return phase == PH_NEWTON && m == 0 && callSetup; }
+  // -------------------------------------------------------------------------
+  // One trip of the state machine, in three parts every lane of a wave shares whatever its
+  // phase: newton_begin (scalars), newton_add for each component of the Newton solution,
+  // and trip_end, whose scalar decisions are followed by one pass over the Nordsieck array.
+  //
+  // What bounded the earlier form was the number of such passes: completing a step, its
+  // new weights, a change of order, the rescaling and the next prediction each read and
+  // wrote the array (8.7 kB per cell and trip on drm19, 510 GB of 1,140 GB per advance of
+  // 128^3), in copies inlined once per path (140 kB of code, twice the instruction cache),
+  // which a wave whose lanes take different paths ran one after another.
+  // -------------------------------------------------------------------------
+  struct Newton {
+    bool on = false;          // this trip's solve gives a Newton iteration
+    bool lin_fail = false;    // a failed linear solve (GMRES): the Newton iteration fails
+    bool conv_fail = false;   // a singular factorisation: the attempt fails
+    bool have = false;        // acor is not zero (its slots are not read otherwise)
+    double sc = 1.0;          // correction for a changed gamma
+    double s = 0.0, sa = 0.0; // sums of (x ewt)^2 and (acor ewt)^2
+  };
 
-  // iteration-matrix set-up at the first evaluation of a Newton attempt: the Jacobian
-  // when stale (or after a convergence failure) and the set-up bookkeeping; the LU of
-  // I - gamma J follows in its own kernel
-  __device__ void setup(const double* y, const double* f, const double Tsol) {
-    const double dgamma = fabs(gamma / gammap - 1.0);
-    const bool jbad = (nst == 0) || (nst >= nstlj + MSBJ) ||
-                      (convfail == FAIL_BAD_J && dgamma < DGMAX_LS) || (convfail == FAIL_OTHER);
-    if (jbad) {
-      ++nje;
-      nstlj = nst;
-      jcur = true;
-      jacobian<M>(y, Tsol, f[N], ws);
-    } else {
-      jcur = false;
-    }
-    ++nsetups;
-    gammap = gamma;          // gamrat = 1 and crate = 1 once the factorisation is in place
-    nstlp = nst;
-    setup_pending = 1;
-  }
-  // after the factorisation: false when it was singular (the attempt is abandoned)
-  __device__ bool after_setup(int sing) {
-    setup_pending = 0;
-    gamrat = 1.0;
-    crate = 1.0;
-    if (sing) {
-      conv_failure();
-      return false;
-    }
-    return true;
-  }
-
-  // one Newton iteration: x solves M x = gamma f(tn, zn0 + acor) - rl1 zn1 - acor (the
-  // right-hand side is formed by the evaluation kernel, the solve by the solve kernel,
-  // with FP64-residual refinement of FP32 factors); returns true when tout is reached
-  __device__ bool iterate() {
+  // start of a trip (its evaluation counted); sing: the flag of a pending factorisation
+  __device__ __forceinline__ void newton_begin(Newton& nw, const int sing) {
     using MS = MatSlots<N1>;
+    ++nfe;
+    if (setup_pending) {   // the factorisation that the set-up asked for is in place
+      setup_pending = 0;
+      gamrat = 1.0;
+      crate = 1.0;
+      nw.conv_fail = sing != 0;
+    }
+    if (phase != PH_NEWTON || nw.conv_fail) return;
     ++nni;
-    double x[N1];
-#pragma unroll
-    for (int i = 0; i < N1; ++i) x[i] = xs[i];
     if (gmres) {
       // the linear solve failed (no residual reduction, or a reduction without
       // convergence after the first Newton iteration): the Newton iteration fails
-      if (mat[MS::IRF] != 0.0) {
-        nls_fail();
-        return false;
-      }
+      nw.lin_fail = mat[MS::IRF] != 0.0;
+      if (nw.lin_fail) return;
     } else if (lu_mode == LU_FP32_IR && !lu64) {
       nir += (long)mat[MS::IRS];
       if (mat[MS::IRF] != 0.0) {
@@ -954,53 +701,383 @@ struct Lane {
         callSetup = true;
         convfail = NO_FAILURES;
         m = 0;
-#pragma unroll
-        for (int i = 0; i < N1; ++i) ws[S::ACOR + i] = 0.0;
         a1 = 0.0; a2 = 0.0; teval = tn;
-        return false;
+        return;
       }
     }
-    if (!gmres && gamrat != 1.0) {   // matrix-free solves use the current gamma
-      const double sc = 2.0 / (1.0 + gamrat);
-#pragma unroll
-      for (int i = 0; i < N1; ++i) x[i] *= sc;
+    nw.on = true;
+    nw.have = a2 != 0.0;
+    if (!gmres && gamrat != 1.0) nw.sc = 2.0 / (1.0 + gamrat);   // matrix-free solves use the current gamma
+  }
+
+  // component i of x, M x = gamma f(tn, zn0 + acor) - rl1 zn1 - acor: acor += x
+  __device__ __forceinline__ void newton_add(Newton& nw, const int i, double x) const {
+    {
+#pragma clang fp contract(off)
+      x *= nw.sc;   // rounded on its own, whatever it is added to
     }
+    double ac = x;
+    if (nw.have) ac = ws[S::ACOR + i] + x;
+    const double e = ws[S::EWT + i];
+    const double p = x * e, pa = ac * e;
+    nw.s += p * p;
+    nw.sa += pa * pa;
+    ws[S::ACOR + i] = ac;
+  }
+
+  // The rest of the trip; true when tout has been reached (the solution there is then in
+  // the zn0 slots, `finite` telling whether it is a number).  The tolerances are read from
+  // the call's arguments (uniform over the cells), never through a stored address.
+  __device__ __forceinline__ bool trip_end(const ReactArgs& a, const Newton& nw, bool& finite) {
+    bool att = false;                                  // an attempt of a step starts
+    bool rescale = false;                              // with h changed by eta
+    bool undo = false, done = false;                   // the prediction taken back; the step completed
+    bool keep = false;                                 // zn(qmax) = acor
+    bool begin = false, restart = false;               // the first attempt; one from zn1 = h f
+    bool reached = false, conv_fail = nw.conv_fail;
+    int adj = 0;
+    double A1 = 0.0, sfac = 0.0;
+    double lc[LMAX], la[LMAX];
 #pragma unroll
-    for (int i = 0; i < N1; ++i) ws[S::ACOR + i] += x[i];
-    const double del = wrms_reg(x);
-    if (m > 0) crate = fmax(CRDOWN * crate, del / delp);
-    // A learned iterate starts farther from the BDF solution than the Nordsieck
-    // prediction, so the iteration stops closer to the convergence threshold: its test
-    // is PRED_NLS_TIGHTEN times stricter, and its first correction (no convergence-rate
-    // history) is never taken as converged
-    const double dcon = del * fmin(1.0, crate) / (pred_state == 2 ? PRED_NLS_TIGHTEN * tq[4] : tq[4]);
-    if (dcon <= 1.0 && !(m == 0 && pred_state == 2)) {
-      // with a learned initial iterate acor is not the first correction alone
-      acnrm = (m == 0 && pred_state != 2) ? del : wrms_ws(S::ACOR);
-      jcur = false;
-      return after_converged();
+    for (int j = 0; j < LMAX; ++j) lc[j] = la[j] = 0.0;
+    const int q0 = q;
+
+    if (nw.on || nw.lin_fail) {
+      bool nls_fail = nw.lin_fail, converged = false;
+      if (nw.on) {
+        const double del = sqrt(nw.s / N1);
+        if (m > 0) crate = fmax(CRDOWN * crate, del / delp);
+        // A learned iterate starts farther from the BDF solution than the Nordsieck
+        // prediction, so the iteration stops closer to the convergence threshold: its test
+        // is PRED_NLS_TIGHTEN times stricter, and its first correction (no convergence-rate
+        // history) is never taken as converged
+        const double dcon = del * fmin(1.0, crate) / (pred_state == 2 ? PRED_NLS_TIGHTEN * tq[4] : tq[4]);
+        if (dcon <= 1.0 && !(m == 0 && pred_state == 2)) {
+          // with a learned initial iterate acor is not the first correction alone
+          acnrm = (m == 0 && pred_state != 2) ? del : sqrt(nw.sa / N1);
+          jcur = false;
+          converged = true;
+        } else if (m >= 1 && del > RDIV * delp) {
+          nls_fail = true;
+        } else {
+          delp = del;
+          ++m;
+          if (m >= MAXCOR) {
+            nls_fail = true;
+          } else {
+            a1 = 0.0; a2 = 1.0; teval = tn;
+          }
+        }
+      }
+      if (nls_fail) {
+        if (pred_state == 2) {
+          // the learned initial iterate did not converge: retry the same step from the
+          // Nordsieck prediction (the matrix set up in this attempt stays valid)
+          ++npredfb;
+          pred_state = 3;
+          callSetup = false;
+          m = 0;
+          a1 = 0.0; a2 = 0.0; teval = tn;
+        } else if (!jcur && !gmres) {
+          callSetup = true;
+          convfail = FAIL_BAD_J;
+          m = 0;
+          a1 = 0.0; a2 = 0.0; teval = tn;
+        } else {
+          conv_fail = true;
+        }
+      }
+      if (converged) {   // error test, then complete the step or retry
+        dsm = acnrm * tq[2];
+        const double etaq = eta_of(BIAS2, dsm, (double)L);
+        if (!(dsm <= 1.0)) {   // a NaN norm fails the test, as in CVODE
+          ++nef;
+          ++netf;
+          nflag = PREV_ERR_FAIL;
+          if (nef == MXNEF) { finish(ST_ERR_FAIL); return false; }
+          undo = true;
+          tn = saved_t;
+          etamax = 1.0;
+          if (nef <= MXNEF1) {
+            eta = fmax(ETAMIN, etaq);
+            if (nef >= SMALL_NEF) eta = fmin(eta, ETAMXF);
+            att = rescale = true;
+          } else if (q > 1) {
+            eta = ETAMIN;
+            adj = -1;
+            att = rescale = true;
+          } else {
+            eta = ETAMIN;
+            h *= eta;
+            hscale = h;
+            qwait = LONG_WAIT;
+            phase = PH_RESTART_F;
+            a1 = 0.0; a2 = 0.0; teval = tn;
+          }
+        } else {
+          done = true;
+          ++nst;
+          for (int i = q; i >= 2; --i) tau[i] = tau[i - 1];
+          if (q == 1 && nst > 1) tau[2] = tau[1];
+          tau[1] = h;
+#pragma unroll
+          for (int j = 0; j < LMAX; ++j) lc[j] = (j <= q) ? l[j] : 0.0;
+          --qwait;
+          if (qwait == 1 && q != qmax) {
+            keep = true;
+            saved_tq5 = tq[5];
+          }
+          const double lq = l[q];
+          const bool rise = choose_next(etaq, [&](const double cquot, double& sq, double& sd) {
+#pragma unroll PASS_UNROLL
+            for (int i = 0; i < N1; ++i) {
+              const double e = ws[S::EWT + i], ac = ws[S::ACOR + i];
+              const double p = (zn(q, i) + lq * ac) * e;
+              sq += p * p;
+              const double d = (ac - cquot * zn(qmax, i)) * e;
+              sd += d * d;
+            }
+          });
+          etamax = (nst <= SMALL_NST) ? ETAMX2 : ETAMX3;
+          ++nstloc;
+          if ((tn - tout) * h >= 0.0) {
+            // CV_NORMAL output: the Nordsieck array interpolated back to tout
+            reached = true;
+            sfac = (tout - tn) / h;
+          } else {
+            if (nstloc >= mxstep) { finish(ST_TOO_MUCH_WORK); return false; }
+            saved_t = tn;
+            ncf = nef = 0;
+            nflag = FIRST_CALL;
+            att = true;
+            rescale = hprime != h;
+            if (rescale && qprime != q) adj = qprime - q;
+            if (rise && adj == 0) keep = true;
+          }
+        }
+        if (adj > 0) A1 = increase_coeffs();
+        if (adj < 0) decrease_coeffs();
+        if (adj != 0) {
+#pragma unroll
+          for (int j = 2; j < LMAX; ++j) la[j] = (j < q || (j == q && adj > 0)) ? l[j] : 0.0;
+        }
+      }
+    } else if (!conv_fail) {
+      if (phase == PH_INIT_F0) {   // the first right-hand side, f(0, y0)
+        double hub_inv = 0.0;
+#pragma unroll PASS_UNROLL
+        for (int i = 0; i < N1; ++i) {
+          const double f = ws[S::F + i];
+          zn(1, i) = f;
+          const double t1 = HUB_FACTOR * fabs(zn(0, i)) + a.atol[i];
+          hub_inv = fmax(hub_inv, fabs(f) / t1);
+        }
+        const double tdist = tout;
+        const double tround = UROUND * tout;
+        if (tdist < 2.0 * tround) { finish(ST_TOO_CLOSE); return false; }
+        hlb = HLB_FACTOR * tround;
+        hub = HUB_FACTOR * tdist;
+        if (hub * hub_inv > 1.0) hub = 1.0 / hub_inv;
+        hg = sqrt(hlb * hub);
+        if (hub < hlb) {
+          h = hg;
+          begin = true;
+        } else {
+          count1 = 1;
+          phase = PH_HIN;
+          a1 = hg; a2 = 0.0; teval = hg;
+        }
+      } else if (phase == PH_HIN) {
+        double s = 0.0;
+#pragma unroll PASS_UNROLL
+        for (int i = 0; i < N1; ++i) {
+          const double d = (ws[S::F + i] - zn(1, i)) / hg * ws[S::EWT + i];
+          s += d * d;
+        }
+        const double yddnrm = sqrt(s / N1);
+        hnew = (yddnrm * hub * hub > 2.0) ? sqrt(2.0 / yddnrm) : sqrt(hg * hub);
+        const double hrat = hnew / hg;
+        begin = count1 == HIN_ITERS || (hrat > 0.5 && hrat < 2.0);
+        if (!begin && count1 > 1 && hrat > 2.0) {
+          hnew = hg;
+          begin = true;
+        }
+        if (begin) {
+          double h0 = H_BIAS * hnew;
+          if (h0 < hlb) h0 = hlb;
+          if (h0 > hub) h0 = hub;
+          h = h0;
+        } else {
+          hg = hnew;
+          ++count1;
+          a1 = hg; a2 = 0.0; teval = hg;
+        }
+      } else if (phase == PH_RESTART_F) {
+        restart = att = true;
+      }
+      if (begin) {
+        hscale = h;
+        hprime = h;
+        nstloc = 0;
+        saved_t = tn;
+        ncf = nef = 0;
+        nflag = FIRST_CALL;
+        att = true;
+      }
     }
-    if (m >= 1 && del > RDIV * delp) {
-      nls_fail();
+    if (conv_fail) {
+      ++ncfn;
+      ++ncf;
+      etamax = 1.0;
+      if (ncf == MXNCF) { finish(ST_CONV_FAIL); return false; }
+      undo = true;
+      tn = saved_t;
+      eta = ETACF;
+      nflag = PREV_CONV_FAIL;
+      att = rescale = true;
+    }
+    if (!(att || undo || done)) return false;
+
+    // the pass: take back or complete, new weights, change the order, rescale, predict;
+    // columns above the order are zero in z, so the triangular sums need no masks
+    const int q1 = q0 + adj;
+    const bool scale = rescale || begin || restart, weights = done && !reached;
+    double fac[LMAX];
+    fac[0] = 1.0;
+    fac[1] = (begin || restart) ? h : eta;
+#pragma unroll
+    for (int j = 2; j < LMAX; ++j) fac[j] = fac[j - 1] * eta;
+    double sn = 0.0;
+    finite = true;
+#pragma unroll PASS_UNROLL
+    for (int i = 0; i < N1; ++i) {
+      double z[LMAX];
+#pragma unroll
+      for (int j = 0; j < LMAX; ++j) z[j] = (j <= q0) ? zn(j, i) : 0.0;
+      if (restart) z[1] = ws[S::F + i];
+      if (undo) {
+#pragma unroll
+        for (int k = 1; k < LMAX; ++k)
+#pragma unroll
+          for (int j = LMAX - 1; j >= k; --j) z[j - 1] -= z[j];
+      }
+      if (done) {
+        const double ac = ws[S::ACOR + i];
+#pragma unroll
+        for (int j = 0; j < LMAX; ++j) z[j] += lc[j] * ac;
+        if (keep) zn(qmax, i) = ac;
+        if (weights) {
+          const double e = 1.0 / (rtol * fabs(z[0]) + a.atol[i]);
+          ws[S::EWT + i] = e;
+          const double p = z[0] * e;
+          sn += p * p;
+        }
+        if (adj > 0) {
+          double zl;
+          {
+#pragma clang fp contract(off)
+            zl = A1 * ac;
+          }
+#pragma unroll
+          for (int j = 2; j < LMAX; ++j) {
+            z[j] += la[j] * zl;
+            if (j == q1) z[j] = zl;
+          }
+        }
+      }
+      if (begin) {
+        const double p = z[0] * ws[S::EWT + i];
+        sn += p * p;
+      }
+      if (adj < 0) {
+        double zq = z[2];
+#pragma unroll
+        for (int j = 3; j < LMAX; ++j) zq = (j == q0) ? z[j] : zq;
+#pragma unroll
+        for (int j = 2; j < LMAX; ++j) {
+          z[j] -= la[j] * zq;
+          if (j == q0) z[j] = 0.0;
+        }
+      }
+      if (reached) {
+        double yo = z[LMAX - 1];
+#pragma unroll
+        for (int j = LMAX - 2; j >= 0; --j) yo = z[j] + sfac * yo;
+        finite = finite && isfinite(yo);
+        z[0] = yo;
+      }
+      if (att) {
+        if (use_pred) ws[S::TMP + i] = z[0];
+        if (scale) {
+#pragma clang fp contract(off)
+#pragma unroll
+          for (int j = 1; j < LMAX; ++j) z[j] *= fac[j];
+        }
+#pragma unroll
+        for (int k = 1; k < LMAX; ++k)
+#pragma unroll
+          for (int j = LMAX - 1; j >= k; --j) z[j - 1] += z[j];
+      }
+#pragma unroll
+      for (int j = 0; j < LMAX; ++j)
+        if (j <= q1) zn(j, i) = z[j];
+    }
+    if (reached) return true;
+    if ((weights || begin) && UROUND * sqrt(sn / N1) > 1.0) {
+      finish(ST_TOO_MUCH_ACC);
       return false;
     }
-    delp = del;
-    ++m;
-    if (m >= MAXCOR) {
-      nls_fail();
-      return false;
+    if (!att) return false;
+    if (adj != 0) {
+      q = q1;
+      L = q + 1;
+      qwait = L;
     }
-    a1 = 0.0; a2 = 1.0; teval = tn;
+    // the attempt: step size, coefficients, Newton set-up.  With the predictor, the state
+    // at tn before the prediction (saved above) is the network's input.
+    pred_state = use_pred ? 1 : 0;
+    if (rescale) {
+      h = hscale * eta;
+      hscale = h;
+    }
+    tn += h;
+    set_coeffs();
+    convfail = (nflag == FIRST_CALL || nflag == PREV_ERR_FAIL) ? NO_FAILURES : FAIL_OTHER;
+    callSetup = (nflag == PREV_CONV_FAIL) || (nflag == PREV_ERR_FAIL) || (nst == 0) ||
+                (nst >= nstlp + MSBP) || (fabs(gamrat - 1.0) > DGMAX);
+    if (gmres) {   // no set-up function: nothing to refresh, the rate estimate restarts
+      callSetup = false;
+      crate = 1.0;
+    }
+    m = 0;
+    a1 = 0.0; a2 = 0.0; teval = tn;
+    phase = PH_NEWTON;
     return false;
   }
 
-  __device__ void restart_f(const double* f) {
-#pragma unroll
-    for (int i = 0; i < N1; ++i) zn(1, i) = h * f[i];
-    attempt(false);
-  }
+  __device__ bool needs_setup() const { return phase == PH_NEWTON && m == 0 && callSetup; }
 
-  __device__ void init_cell(const double* y0) {
+  // iteration-matrix set-up at the first evaluation of a Newton attempt: the Jacobian
+  // when stale (or after a convergence failure) and the set-up bookkeeping; the LU of
+  // I - gamma J follows in its own kernel.  The Jacobian goes to the slots of tile `js`.
+  __device__ void setup(const double* y, const double fT, const double Tsol, const WS& js) {
+    const double dgamma = fabs(gamma / gammap - 1.0);
+    const bool jbad = (nst == 0) || (nst >= nstlj + MSBJ) ||
+                      (convfail == FAIL_BAD_J && dgamma < DGMAX_LS) || (convfail == FAIL_OTHER);
+    if (jbad) {
+      ++nje;
+      nstlj = nst;
+      jcur = true;
+      jacobian<M>(y, Tsol, fT, ws, js);
+    } else {
+      jcur = false;
+    }
+    ++nsetups;
+    gammap = gamma;          // gamrat = 1 and crate = 1 once the factorisation is in place
+    nstlp = nst;
+    setup_pending = 1;
+  }
+  __device__ __forceinline__ void init_cell(const ReactArgs& a, const double* y0) {
     tn = 0.0;
     q = 1; L = 2; qwait = L; qprime = 1;
     etamax = ETAMX1;
@@ -1021,12 +1098,7 @@ struct Lane {
     for (int j = 0; j < LMAX; ++j)
 #pragma unroll
       for (int i = 0; i < N1; ++i) zn(j, i) = (j == 0) ? y0[i] : 0.0;
-    // the first evaluations (f0 and the initial-step search) form zn0 + a1 zn1 + a2 acor
-    // with a2 = 0: acor must hold numbers, since 0 x NaN is NaN in whatever the
-    // workspace held before
-#pragma unroll
-    for (int i = 0; i < N1; ++i) ws[S::ACOR + i] = 0.0;
-    ewtset();
+    ewtset(a);
     status = ST_OK;
     phase = PH_INIT_F0;
     setup_pending = 0;
@@ -1078,7 +1150,6 @@ __device__ __forceinline__ void load_lane(Lane<M>& st, const ReactArgs& a, long 
   st.ws = w;
   st.iws = cell_iws<M>(a.iws, c);
   st.mat = cell_mat<M>(a.mat, c);
-  st.xs = &st.mat[MatSlots<M::N1>::X];
   st.qmax = a.qmax;
   st.lu_mode = a.lu_mode;
   st.ir_sweeps = a.ir_sweeps;
@@ -1111,25 +1182,60 @@ __device__ __forceinline__ T lane_field(const WS& w, size_t off) {
 }
 #define LANE_FIELD(M, w, f) lane_field<M, decltype(Lane<M>::f)>((w), offsetof(Lane<M>, f))
 
-// Copies between 64 lanes' rows in LDS (sm[l * LEN + i], lane l's cell cells[l], or -1)
-// and the cell-major region: consecutive lanes of a store or load handle consecutive
-// words of one cell's row, so each instruction touches a few whole lines instead of
-// one line per lane.  Called by all 64 threads of a one-wave block.
-template <int LEN>
+// f(std::integral_constant<int, k>) for k = 0 .. N-1, each call with k a compile-time
+// constant (so arrays indexed by k stay in registers however long the sequence)
+template <class F, int... K>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, K...>) {
+  (f(std::integral_constant<int, K>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
+
+// Copies between 64 lanes' rows in LDS (word i of lane l's row at sm[l * LD + i], l's
+// cell cells[l], or -1) and LEN words of the cell-major region: consecutive lanes of a
+// store or load handle consecutive words of one cell's row, so each instruction touches a
+// few whole lines instead of one line per lane.  Called by all 64 threads of a one-wave
+// block.
+template <int LEN, int LD = LEN>
 __device__ __forceinline__ void rows_to_cells(const double* sm, const long* cells, double* mat, long stride, int off) {
   for (int e = threadIdx.x; e < 64 * LEN; e += 64) {
     const int l = e / LEN, i = e - l * LEN;
     const long c = cells[l];
-    if (c >= 0) mat[c * stride + off + i] = sm[l * LEN + i];
+    if (c >= 0) mat[c * stride + off + i] = sm[l * LD + i];
   }
 }
-template <int LEN>
+template <int LEN, int LD = LEN>
 __device__ __forceinline__ void cells_to_rows(double* sm, const long* cells, const double* mat, long stride, int off) {
   for (int e = threadIdx.x; e < 64 * LEN; e += 64) {
     const int l = e / LEN, i = e - l * LEN;
     const long c = cells[l];
-    sm[l * LEN + i] = (c >= 0) ? mat[c * stride + off + i] : 0.0;
+    sm[l * LD + i] = (c >= 0) ? mat[c * stride + off + i] : 0.0;
   }
+}
+// Vectors of N1 words pass through LDS in windows of W words, lane rows an odd number of
+// words apart (no bank conflicts): whole up to 32 unknowns, 16 at a time beyond, where a
+// whole row per lane (28 kB at 54 unknowns, 46 kB at 89) would leave a CU 5 or 3 waves.
+template <int N1>
+struct Window {
+  static constexpr int W = N1 <= 32 ? N1 : 16;
+  static constexpr int LD = W | 1;
+  static constexpr int COUNT = (N1 + W - 1) / W;
+};
+// window w (a compile-time constant) of a cell's N1-word vector at word `off` of the
+// matrix region
+template <int N1, int w>
+__device__ __forceinline__ void window_to_cells(const double* sm, const long* cells, double* mat, long stride, int off) {
+  using V = Window<N1>;
+  constexpr int LEN = (w + 1) * V::W <= N1 ? V::W : N1 - w * V::W;
+  rows_to_cells<LEN, V::LD>(sm, cells, mat, stride, off + w * V::W);
+}
+template <int N1, int w>
+__device__ __forceinline__ void window_from_cells(double* sm, const long* cells, const double* mat, long stride, int off) {
+  using V = Window<N1>;
+  constexpr int LEN = (w + 1) * V::W <= N1 ? V::W : N1 - w * V::W;
+  cells_to_rows<LEN, V::LD>(sm, cells, mat, stride, off + w * V::W);
 }
 
 // ---------------------------------------------------------------------------
@@ -1195,7 +1301,7 @@ __global__ void __launch_bounds__(64) k_init(const ReactArgs a) {
     st.ws = w;
     st.iws = cell_iws<M>(a.iws, c);
     st.mat = cell_mat<M>(a.mat, c);
-    st.qmax = a.qmax;
+      st.qmax = a.qmax;
     st.lu_mode = a.lu_mode;
     st.ir_sweeps = a.ir_sweeps;
     st.use_pred = a.use_pred;
@@ -1212,8 +1318,6 @@ __global__ void __launch_bounds__(64) k_init(const ReactArgs a) {
       st.pred_state = 0;
       if (a.cell_status) a.cell_status[slot_cell(a, c)] = 0;
     } else {
-#pragma unroll
-      for (int i = 0; i < N1; ++i) w[S::ATOL + i] = a.atol[i];
       double y0[N1];
 #pragma unroll
       for (int k = 0; k < N; ++k) {
@@ -1223,7 +1327,7 @@ __global__ void __launch_bounds__(64) k_init(const ReactArgs a) {
       y0[N] = a.T.p[cell_off(a.T, ci, cj, ck)];
       st.rE0 = a.rE.p[cell_off(a.rE, ci, cj, ck)];
       st.fH = a.rEsrc.p ? a.rEsrc.p[cell_off(a.rEsrc, ci, cj, ck)] : 0.0;
-      st.init_cell(y0);
+      st.init_cell(a, y0);
       active = true;
     }
     store_lane(st, w);
@@ -1238,12 +1342,14 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(PELE_EVAL_WAVES(M::N1)) 
   constexpr int N1 = M::N1;
   using S = Slots<N1>;
   using MS = MatSlots<N1>;
-  __shared__ double sB[64 * N1];
+  using V = Window<N1>;
+  __shared__ double sB[64 * V::LD];
   __shared__ long scell[64];
   const long idx = (long)blockIdx.x * 64 + threadIdx.x;
   int iters = 0;
-  bool newton = false;
+  bool newton = false, due = false;   // due: the solve kernel's (a set-up's first solve may come with its factors)
   long c = -1;
+  double f[N1];
   if (idx < (long)*count) {
     c = list[idx];
     const WS w = cell_ws<M>(a.ws, c);
@@ -1251,39 +1357,58 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(PELE_EVAL_WAVES(M::N1)) 
     const int phase = LANE_FIELD(M, w, phase);
     if (phase != PH_NEED_CELL) {
       const double a1 = LANE_FIELD(M, w, a1), a2 = LANE_FIELD(M, w, a2);
-      double y[N1], f[N1], Tsol;
-#pragma unroll
-      for (int i = 0; i < N1; ++i) y[i] = w[S::ZN + i] + a1 * w[S::ZN + N1 + i] + a2 * w[S::ACOR + i];
-      rhs<M>(y, LANE_FIELD(M, w, teval), w, LANE_FIELD(M, w, rE0), LANE_FIELD(M, w, fH), f, Tsol, &iters);
+      const bool has_ac = a2 != 0.0;   // the acor slots are read only where they count
+      double y[N1], Tsol;
 #pragma unroll
       for (int i = 0; i < N1; ++i) {
-        w[S::Y + i] = y[i];
-        w[S::F + i] = f[i];
+        const double ac = has_ac ? w[S::ACOR + i] : 0.0;
+        y[i] = w[S::ZN + i] + a1 * w[S::ZN + N1 + i] + a2 * ac;
       }
-      w[S::TS] = Tsol;
-      if (phase == PH_NEWTON) {
+      rhs<M>(y, LANE_FIELD(M, w, teval), w, LANE_FIELD(M, w, rE0), LANE_FIELD(M, w, fH), f, Tsol, &iters);
+      newton = phase == PH_NEWTON;
+      const bool setup = newton && LANE_FIELD(M, w, m) == 0 && LANE_FIELD(M, w, callSetup);
+      if (!newton || setup || a.gmres) {
+        // the point and its right-hand side, for a Jacobian, the matrix-free solve and the
+        // phases outside the Newton iteration (an iteration consumes the solution instead)
+#pragma unroll
+        for (int i = 0; i < N1; ++i) {
+          w[S::Y + i] = y[i];
+          w[S::F + i] = f[i];
+        }
+        w[S::TS] = Tsol;
+      }
+      if (newton) {
         // the Newton system's right-hand side gamma f - rl1 zn1 - acor
-        newton = true;
+        due = !(a.fuse && setup);
         const double gamma = LANE_FIELD(M, w, gamma), rl1 = LANE_FIELD(M, w, rl1);
 #pragma unroll
-        for (int i = 0; i < N1; ++i) f[i] = gamma * f[i] - rl1 * w[S::ZN + N1 + i] - w[S::ACOR + i];
+        for (int i = 0; i < N1; ++i) {
+          const double ac = has_ac ? w[S::ACOR + i] : 0.0;
+          f[i] = gamma * f[i] - rl1 * w[S::ZN + N1 + i] - ac;
+        }
         if (a.lu_lane) {
           const CM mat = cell_mat<M>(a.mat, c);
 #pragma unroll
           for (int i = 0; i < N1; ++i) mat[MS::B + i] = f[i];
-        } else {
-#pragma unroll
-          for (int i = 0; i < N1; ++i) sB[threadIdx.x * N1 + i] = f[i];
         }
       }
     }
   }
   if (!a.lu_lane) {
     scell[threadIdx.x] = newton ? c : -1;
-    __syncthreads();
-    rows_to_cells<N1>(sB, scell, a.mat, MS::STRIDE, MS::B);
+    static_for<V::COUNT>([&](auto wc) {
+      constexpr int w0 = decltype(wc)::value * V::W;
+      __syncthreads();
+      if (newton) {
+#pragma unroll
+        for (int i = 0; i < V::W; ++i)
+          if (w0 + i < N1) sB[threadIdx.x * V::LD + i] = f[w0 + i];
+      }
+      __syncthreads();
+      window_to_cells<N1, decltype(wc)::value>(sB, scell, a.mat, MS::STRIDE, MS::B);
+    });
   }
-  wave_append(newton, (int)c, a.nlist, &a.counts[6]);
+  wave_append(due, (int)c, a.nlist, &a.counts[6]);
   if (a.counters) wave_add(&a.counters[CNT_HY2T], (unsigned long long)iters);
 }
 
@@ -1294,9 +1419,15 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(PELE_SETUP_WAVES(M::N1))
   constexpr int N1 = M::N1;
   using S = Slots<N1>;
   using MS = MatSlots<N1>;
-  __shared__ double sJ[64 * N1];
+  using V = Window<N1>;
+  __shared__ double sJ[64 * V::LD];
   __shared__ long scell[64];
   const long idx = (long)blockIdx.x * 64 + threadIdx.x;
+  // The new Jacobian is staged in the JS slots of tile `idx`, not of the cell's own tile:
+  // the set-up list scatters a wave's cells over many tiles, where each 8-byte store would
+  // touch a line of its own; by list position a wave's stores and loads are whole lines.
+  // (No other kernel of a trip keeps anything in these slots; GMRES, which does, has no set-up.)
+  const WS wj = cell_ws<M>(a.ws, idx < (long)*count ? idx : 0);
   long c = -1;
   bool fresh = false;   // this lane evaluated a new Jacobian
   if (idx < (long)*count) {
@@ -1305,38 +1436,37 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(PELE_SETUP_WAVES(M::N1))
     Lane<M> st;
     load_lane(st, a, c);
     if (st.needs_setup() && !st.setup_pending) {
-      double y[N1], f[N1];
+      double y[N1];
 #pragma unroll
-      for (int i = 0; i < N1; ++i) {
-        y[i] = w[S::Y + i];
-        f[i] = w[S::F + i];
-      }
-      st.setup(y, f, w[S::TS]);
+      for (int i = 0; i < N1; ++i) y[i] = w[S::Y + i];
+      st.setup(y, w[S::F + N1 - 1], w[S::TS], wj);
       fresh = st.jcur;
       store_lane(st, w);
     }
   }
-  // the Jacobian (accumulated in the wave-tiled slots) goes to the matrix region, where
-  // the factorisation and refinement kernels read it row by row
+  // the Jacobian goes to the matrix region, where the factorisation and refinement kernels
+  // read it row by row
   if (a.lu_lane) {
     if (fresh) {
-      const WS w = cell_ws<M>(a.ws, c);
       const CM mat = cell_mat<M>(a.mat, c);
 #pragma unroll 1
-      for (int e = 0; e < N1 * N1; ++e) mat[MS::JS + e] = w[S::JS + e];
+      for (int e = 0; e < N1 * N1; ++e) mat[MS::JS + e] = wj[S::JS + e];
     }
   } else {
     scell[threadIdx.x] = fresh ? c : -1;
-    const WS w = cell_ws<M>(a.ws, fresh ? c : 0);
 #pragma unroll 1
     for (int r = 0; r < N1; ++r) {
-      __syncthreads();
-      if (fresh) {
+      static_for<V::COUNT>([&](auto wc) {
+        constexpr int w0 = decltype(wc)::value * V::W;
+        __syncthreads();
+        if (fresh) {
 #pragma unroll
-        for (int j = 0; j < N1; ++j) sJ[threadIdx.x * N1 + j] = w[S::JS + r * N1 + j];
-      }
-      __syncthreads();
-      rows_to_cells<N1>(sJ, scell, a.mat, MS::STRIDE, MS::JS + r * N1);
+          for (int j = 0; j < V::W; ++j)
+            if (w0 + j < N1) sJ[threadIdx.x * V::LD + j] = wj[S::JS + r * N1 + w0 + j];
+        }
+        __syncthreads();
+        window_to_cells<N1, decltype(wc)::value>(sJ, scell, a.mat, MS::STRIDE, MS::JS + r * N1);
+      });
     }
   }
 }
@@ -1458,16 +1588,12 @@ __global__ void __launch_bounds__(64) k_lu_lane(const ReactArgs a, const int* __
 }
 
 
-// f(std::integral_constant<int, k>) for k = 0 .. N-1, each call with k a compile-time
-// constant (so arrays indexed by k stay in registers however long the sequence)
-template <class F, int... K>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, K...>) {
-  (f(std::integral_constant<int, K>{}), ...);
-}
-template <int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
+// Keeps the scheduler from hoisting what follows above this point.
+#if defined(__HIP_DEVICE_COMPILE__)
+#define PELE_SCHED_BARRIER() __builtin_amdgcn_sched_barrier(0)
+#else
+#define PELE_SCHED_BARRIER() ((void)0)
+#endif
 
 // x as held by lane `src` of the wave (src uniform, possibly known only at run time),
 // read with v_readlane: a scalar broadcast, no trip through the LDS crossbar
@@ -1509,6 +1635,61 @@ __device__ __forceinline__ unsigned long long group_max_u64(unsigned long long v
   return (threadIdx.x & 32) ? b : a;
 }
 
+// the same for 32-bit keys: one v_max_u32 per step
+template <int G>
+__device__ __forceinline__ unsigned group_max_u32(unsigned v) {
+  static_assert(G == 32 || G == 64, "a half-wave or the whole wave");
+  auto step = [&](auto ctrl) {
+    constexpr int C = decltype(ctrl)::value;
+    const unsigned o = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, C, 0xF, 0xF, false);
+    v = o > v ? o : v;
+  };
+  step(std::integral_constant<int, 0xB1>{});
+  step(std::integral_constant<int, 0x4E>{});
+  step(std::integral_constant<int, 0x141>{});
+  step(std::integral_constant<int, 0x140>{});
+  const unsigned r0 = (unsigned)__builtin_amdgcn_readlane((int)v, 0), r1 = (unsigned)__builtin_amdgcn_readlane((int)v, 16);
+  const unsigned r2 = (unsigned)__builtin_amdgcn_readlane((int)v, 32), r3 = (unsigned)__builtin_amdgcn_readlane((int)v, 48);
+  const unsigned a = r0 > r1 ? r0 : r1, b = r2 > r3 ? r2 : r3;
+  if (G == 64) return a > b ? a : b;
+  return (threadIdx.x & 32) ? b : a;
+}
+
+// The pivot of a column: the group's lane with the largest |v| among its live lanes, ties
+// to the lowest lane, a NaN counting as infinite.  Returns the lane within the group;
+// `key` is the pivot's magnitude as its bits + 1 (1: every live entry is zero, 0: no live
+// lane).  The bits of non-negative doubles order as integers, so a first search takes the
+// upper words alone (one instruction per DPP step instead of five, and the rows' maxima
+// combine on the scalar unit), and the lower words decide only when several lanes share
+// the largest upper word.  Same choice as a search over all 64 bits; on 22 unknowns the
+// 64-bit one was 60 of a column's 158 vector instructions, which bound the factorisation.
+template <int G>
+__device__ __forceinline__ int group_pivot(const bool live, const double v, unsigned long long& key) {
+  const unsigned long long bits = (unsigned long long)__double_as_longlong(v);
+  const unsigned top = (unsigned)(bits >> 32) & 0x7FFFFFFFu;
+  const unsigned hi = live ? (top < 0x7FF00000u ? top : 0x7FF00000u) + 1u : 0u;
+  const unsigned hmax = group_max_u32<G>(hi);
+  const int half = (G == 32) ? (int)(threadIdx.x & 32) : 0;
+  auto mine = [&](unsigned long long b) { return (G == 64) ? b : (b >> half) & 0xFFFFFFFFull; };
+  const bool cand = hi == hmax;
+  const unsigned long long all = __ballot(cand);
+  const unsigned long long c = mine(all);
+  int who = __ffsll((long long)c) - 1;
+  key = ((unsigned long long)hmax << 32) + 1u;
+  if (hmax != 0u) key -= 1ull << 32;
+  else key = 0ull;
+  // several candidates, or nothing but zeros and numbers below 2^-1042, in some group
+  const bool tie = (c & (c - 1ull)) != 0ull || hmax == 1u;
+  if (__ballot(tie) != 0ull) {
+    const unsigned lo = (cand && hi <= 0x7FF00000u) ? (unsigned)bits : 0u;
+    const unsigned lmax = group_max_u32<G>(lo);
+    const unsigned long long w = mine(__ballot(cand && lo == lmax));
+    who = __ffsll((long long)w) - 1;
+    if (hmax != 0u) key += lmax;
+  }
+  return who;
+}
+
 // x as held by lane `src` (a compile-time constant) of this lane's group of G lanes:
 // v_readlane for a whole-wave group (measured faster than a permute); two groups per
 // wave would need both lanes read and a select, which measured no faster than the
@@ -1539,13 +1720,18 @@ struct Coop {
 // One cell's factorisation by its group of G lanes (lane r of the group holds row r):
 // `work` (uniform over the group) says whether the group factors at all, `mat` is the
 // cell's matrix region; every lane of the wave must call it (it synchronises the block).
+// solve (uniform): the cell's first Newton solve follows from the registers -- the right-hand side B takes the
+// elimination's row operations as one more column (the forward substitution, in the same
+// order and rounding as the solve kernel's), the back substitution walks the pivots from
+// the last -- so that this solve reads no factors (a third of the solves on the stiff mix).
 // Returns 0, or 1 + the first column without a nonzero pivot (uniform over the group).
 template <int N1, class Real>
-__device__ __forceinline__ int lu_coop_core(const CM& mat, const bool work, const double gamma) {
+__device__ __forceinline__ int lu_coop_core(const CM& mat, const bool work, const double gamma,
+                                            const bool solve = false) {
   constexpr int G = Coop<N1>::G, CPW = Coop<N1>::CPW;
   using A = LUAcc<N1, Real>;
   constexpr bool IS32 = sizeof(Real) == 4;
-  __shared__ Real prow[CPW][N1];
+  __shared__ Real prow[CPW][N1 + 1];
   const int lane = threadIdx.x;
   const int half = lane / G, r = lane % G;
   const bool row = work && r < N1;
@@ -1558,52 +1744,42 @@ __device__ __forceinline__ int lu_coop_core(const CM& mat, const bool work, cons
     for (int j = 0; j < N1; ++j) m[j] = (Real)0;
   }
   bool done = !row;
-  int my_step = 0, sing = 0;
+  int my_step = row ? 0 : -1, sing = 0;
+  Real bv = (solve && row) ? (Real)mat[MatSlots<N1>::B + r] : (Real)0, piv = (Real)1;
   static_for<N1>([&](auto kc) {
     constexpr int k = decltype(kc)::value;
-    // Pivot: the largest |m_rk| over the remaining rows, ties to the lowest row.  The
-    // bits of a non-negative double order as unsigned integers, so the search is one
-    // 64-bit max over the cell's lanes and a ballot for the lowest lane holding it;
-    // remaining rows carry bits + 1 so that a zero entry still beats a finished row, and
-    // a NaN row counts as infinite (it still takes a definite place in the order).
-    unsigned long long key = 0ull;
-    if (!done) {
-      double av = fabs((double)m[k]);
-      if (av != av) av = HUGE_VAL;
-      key = (unsigned long long)__double_as_longlong(av) + 1ull;
-    }
-    const unsigned long long kmax = group_max_u64<G>(key);
-    const unsigned long long ball = __ballot(key == kmax);
-    const unsigned long long mine = (G == 64) ? ball : ((ball >> (half * 32)) & 0xFFFFFFFFull);
-    const int who = __ffsll((long long)mine) - 1;
-    const bool nonzero = kmax > 1ull;   // the pivot magnitude is > 0 (equal in all G lanes)
+    // Pivot: the largest |m_rk| over the remaining rows, ties to the lowest row
+    unsigned long long key;
+    const int who = group_pivot<G>(!done, (double)m[k], key);
+    const bool nonzero = key > 1ull;   // the pivot magnitude is > 0 (equal in all G lanes)
     if (!nonzero && sing == 0) sing = k + 1;
+    const bool upd = !done && r != who && nonzero;
     if constexpr (G == 64 && !IS32) {
       // one cell per wave, FP64: the pivot row's entries are read from lane `who`
-      // (uniform) with v_readlane; that lane's row is not updated in this step.  (The
-      // FP32 factorisation measured faster with the LDS broadcast below.)
-      const bool upd = !done && r != who && nonzero;
-      const Real pk = lane_read(m[k], who);
-      Real l = (Real)0;
-      if (upd) {
-        l = m[k] * ((Real)1 / pk);
-        m[k] = l;
-      }
+      // (uniform) with v_readlane.  The multiplier is zero in the lanes whose row stays as
+      // it is, so the updates need no mask (which the compiler makes two selects per
+      // entry).  (The FP32 factorisation measured faster with the LDS broadcast below.)
+      const Real pk = lane_read(m[k], who), pb = lane_read(bv, who);
+      const Real l = upd ? m[k] * ((Real)1 / pk) : (Real)0;
+      if (upd) m[k] = l;
+      bv -= l * pb;
 #pragma unroll
-      for (int j = k + 1; j < N1; ++j) {
+      for (int j = k + 1; j < N1; ++j) {   // in order: hoisted reads cost 60 registers at 54 unknowns
         const Real pj = lane_read(m[j], who);
-        if (upd && l != (Real)0) m[j] -= l * pj;
+        m[j] -= l * pj;
+        PELE_SCHED_BARRIER();
       }
     } else {
       if (row && r == who) {   // the pivot row's columns k.. (those left of k are multipliers)
 #pragma unroll
         for (int j = k; j < N1; ++j) prow[half][j] = m[j];
+        prow[half][N1] = bv;
       }
       __syncthreads();
-      if (!done && r != who && nonzero) {
-        const Real inv = (Real)1 / prow[half][k];
-        const Real l = m[k] * inv;
+      if (upd) {
+        const Real l = m[k] * ((Real)1 / prow[half][k]);
         m[k] = l;
+        bv -= l * prow[half][N1];
         if (l != (Real)0) {
 #pragma unroll
           for (int j = k + 1; j < N1; ++j) m[j] -= l * prow[half][j];
@@ -1614,12 +1790,32 @@ __device__ __forceinline__ int lu_coop_core(const CM& mat, const bool work, cons
     if (r == who && !done) {
       done = true;
       my_step = k;
+      piv = m[k];
     }
   });
   if (row) {
 #pragma unroll
-    for (int j = 0; j < N1; ++j) A::at(mat, my_step * N1 + j) = m[j];
+    for (int j = 0; j < N1; ++j) A::at(mat, my_step, j) = m[j];
     mat.perm(MatSlots<N1>::PERM, my_step) = r;
+  }
+  if constexpr (!IS32) {
+    if (solve) {   // uniform over the block
+      const double inv = 1.0 / piv;
+      static_for<N1>([&](auto kc) {
+        constexpr int k = N1 - 1 - decltype(kc)::value;
+        const unsigned long long ball = __ballot(my_step == k);
+        if (my_step == k) bv *= inv;
+        double xk;
+        if constexpr (G == 64) {
+          xk = lane_read(bv, (__ffsll((long long)ball) - 1) & 63);
+        } else {
+          // (a group without a cell has no such lane: any of its lanes will do)
+          xk = __shfl(bv, (__ffsll((long long)((ball >> (half * 32)) & 0xFFFFFFFFull)) - 1) & (G - 1), G);
+        }
+        if (my_step < k) bv -= m[k] * xk;
+      });
+      if (row && sing == 0) mat[MatSlots<N1>::X + my_step] = bv;
+    }
   }
   __syncthreads();   // prow is reused by the next group of this block
   return sing;
@@ -1653,7 +1849,7 @@ __device__ __forceinline__ void lu_coop_pair(const ReactArgs& a, const int* __re
     work = pend && (fp32_cell == IS32);
     gamma = LANE_FIELD(M, w, gamma);
   }
-  const int sing = lu_coop_core<N1, Real>(cell_mat<M>(a.mat, c < 0 ? 0 : c), work, gamma);
+  const int sing = lu_coop_core<N1, Real>(cell_mat<M>(a.mat, c < 0 ? 0 : c), work, gamma, a.fuse != 0);
   if (work && r == 0) cell_ws<M>(a.ws, c)[S::SING] = (double)sing;
 }
 
@@ -1838,7 +2034,7 @@ __device__ __forceinline__ int lu_mfma_core(const CM& mat, const bool work, cons
 #pragma unroll 1
   for (int e = l; e < N1 * N1; e += 64) {
     const int s = e / N1, j = e - (e / N1) * N1;
-    A::at(mat, e) = sm[sstep[s] * LD + j];
+    A::at(mat, s, j) = sm[sstep[s] * LD + j];
   }
   if (l < N1) mat.perm(MS::PERM, l) = sstep[l];
   __syncthreads();   // the LDS is reused by the next cell of this block
@@ -1956,12 +2152,14 @@ __device__ __forceinline__ void solve_coop_core(const CM& mat, const bool work, 
   int pr = 0;
   if (row) {
 #pragma unroll
-    for (int j = 0; j < N1; ++j) lrow[j] = A::at(mat, r * N1 + j);
+    for (int j = 0; j < N1; ++j) lrow[j] = A::at(mat, r, j);
     pr = mat.perm(MS::PERM, r);
   } else {
 #pragma unroll
     for (int j = 0; j < N1; ++j) lrow[j] = (Real)0;
   }
+  // one division per lane ahead of the substitution, not one in each step of its chain
+  const double inv = row ? 1.0 / (double)A::at(mat, r, r) : 0.0;
   // x = U^-1 L^-1 (P v) where lane r holds v[PERM[r]] on entry
   auto subst = [&](double xv) {
 #pragma unroll
@@ -1971,7 +2169,7 @@ __device__ __forceinline__ void solve_coop_core(const CM& mat, const bool work, 
     }
 #pragma unroll
     for (int k = N1 - 1; k >= 0; --k) {
-      if (r == k) xv /= (double)lrow[k];
+      if (r == k) xv *= inv;
       const double xk = group_bcast<G>(xv, k);
       if (r < k) xv -= (double)lrow[k] * xk;
     }
@@ -2317,9 +2515,10 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(PELE_CONSUME_WAVES) k_co
                                                 unsigned int* next_count, int* snext, unsigned int* snext_count) {
   constexpr int N = M::NS, N1 = M::N1;
   using S = Slots<N1>;
+  using V = Window<N1>;
   const long idx = (long)blockIdx.x * 64 + threadIdx.x;
   const long n = (long)*count;
-  __shared__ double sX[64 * N1];
+  __shared__ double sX[64 * V::LD];
   __shared__ long scell[64];
   bool keep = false, want_setup = false, want_pred = false;
   unsigned long long t_cells = 0, t_nst = 0, t_nfe = 0, t_nje = 0, t_nsetups = 0, t_nni = 0, t_ncfn = 0,
@@ -2330,71 +2529,46 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(PELE_CONSUME_WAVES) k_co
   }
   const WS w0 = cell_ws<M>(a.ws, c < 0 ? 0 : c);
   const int phase0 = (c >= 0) ? LANE_FIELD(M, w0, phase) : (int)PH_NEED_CELL;
-  if (!a.lu_lane) {
-    // this trip's Newton solutions, read from the matrix region as whole lines
-    scell[threadIdx.x] = (phase0 == PH_NEWTON) ? c : -1;
-    __syncthreads();
-    cells_to_rows<N1>(sX, scell, a.mat, MatSlots<N1>::STRIDE, MatSlots<N1>::X);
-    __syncthreads();
-  }
-  if (phase0 != PH_NEED_CELL) {
-    const WS w = w0;
-    Lane<M> st;
+  const bool act = phase0 != PH_NEED_CELL;
+  const WS w = w0;
+  Lane<M> st;
+  typename Lane<M>::Newton nw;
+  if (act) {
     load_lane(st, a, c);
-    if (!a.lu_lane) st.xs = &sX[threadIdx.x * N1];
-    {
-      ++st.nfe;
-      // the right-hand side at this trip's point is read only by the phases that use it
-      // (a Newton iteration consumes the solve's result instead)
-      double f[N1];
-      auto load_f = [&]() {
+    st.newton_begin(nw, (st.setup_pending && w[S::SING] != 0.0) ? 1 : 0);
+  }
+  if (a.lu_lane) {
+    if (nw.on) {
 #pragma unroll
-        for (int i = 0; i < N1; ++i) f[i] = w[S::F + i];
-      };
-      bool reached = false;
-      bool proceed = true;
-      if (st.setup_pending) proceed = st.after_setup((int)w[S::SING]);
-      if (proceed) {
-        switch (st.phase) {
-          case PH_INIT_F0:
+      for (int i = 0; i < N1; ++i) st.newton_add(nw, i, st.mat[MatSlots<N1>::X + i]);
+    }
+  } else {
+    // this trip's Newton solutions, read from the matrix region as whole lines
+    scell[threadIdx.x] = nw.on ? c : -1;
+    static_for<V::COUNT>([&](auto wc) {
+      constexpr int w0i = decltype(wc)::value * V::W;
+      __syncthreads();
+      window_from_cells<N1, decltype(wc)::value>(sX, scell, a.mat, MatSlots<N1>::STRIDE, MatSlots<N1>::X);
+      __syncthreads();
+      if (nw.on) {
 #pragma unroll
-            for (int i = 0; i < N1; ++i) st.zn(1, i) = w[S::F + i];
-            st.after_f0();
-            break;
-          case PH_HIN:
-            load_f();
-            st.after_hin(f);
-            break;
-          case PH_NEWTON:
-            reached = st.iterate();
-            break;
-          case PH_RESTART_F:
-            load_f();
-            st.restart_f(f);
-            break;
-          default:
-            break;
-        }
+        for (int i = 0; i < V::W; ++i)
+          if (w0i + i < N1) st.newton_add(nw, w0i + i, sX[threadIdx.x * V::LD + i]);
       }
+    });
+  }
+  if (act) {
+    {
+      bool finite = true;
+      const bool reached = st.trip_end(a, nw, finite);
       int ci, cj, ck;
       slot_ijk(a, c, ci, cj, ck);
       if (reached) {
-        // CV_NORMAL output: interpolate the Nordsieck array back to tout
-        const double sfac = (st.tout - st.tn) / st.h;
-        double yo[N1];
-#pragma unroll
-        for (int i = 0; i < N1; ++i) yo[i] = st.zn(st.q, i);
-        for (int j = st.q - 1; j >= 0; --j)
-#pragma unroll
-          for (int i = 0; i < N1; ++i) yo[i] = st.zn(j, i) + sfac * yo[i];
-        bool finite = true;
-#pragma unroll
-        for (int i = 0; i < N1; ++i) finite = finite && isfinite(yo[i]);
         st.finish(finite ? ST_OK : ST_NONFINITE);
         if (finite) {
 #pragma unroll
-          for (int k = 0; k < N; ++k) a.rY.p[cell_off(a.rY, ci, cj, ck) + k * a.rY.ns] = yo[k];
-          a.T.p[cell_off(a.T, ci, cj, ck)] = yo[N];
+          for (int k = 0; k < N; ++k) a.rY.p[cell_off(a.rY, ci, cj, ck) + k * a.rY.ns] = st.zn(0, k);
+          a.T.p[cell_off(a.T, ci, cj, ck)] = st.zn(0, N);
           a.rE.p[cell_off(a.rE, ci, cj, ck)] = st.rE0 + st.fH * st.tout;
         }
       }
@@ -2545,7 +2719,6 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(OCC) k_persist(const Rea
   st.ws = w;
   st.iws = cell_iws<M>(a.iws, slot);
   st.mat = mat;
-  st.xs = &stage[lane * N1];
   st.qmax = a.qmax;
   st.lu_mode = a.lu_mode;
   st.ir_sweeps = a.ir_sweeps;
@@ -2600,8 +2773,6 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(OCC) k_persist(const Rea
             }
           }
           if (cell >= 0) {
-#pragma unroll
-            for (int i = 0; i < N1; ++i) w[S::ATOL + i] = a.atol[i];
             double y0[N1];
 #pragma unroll
             for (int k = 0; k < N; ++k) {
@@ -2611,7 +2782,7 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(OCC) k_persist(const Rea
             y0[N] = a.T.p[cell_off(a.T, ci, cj, ck)];
             st.rE0 = a.rE.p[cell_off(a.rE, ci, cj, ck)];
             st.fH = a.rEsrc.p ? a.rEsrc.p[cell_off(a.rEsrc, ci, cj, ck)] : 0.0;
-            st.init_cell(y0);
+            st.init_cell(a, y0);
             trips = 0;
           }
         }
@@ -2630,14 +2801,21 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(OCC) k_persist(const Rea
     bool newton = false;
     if (act) {
       int it = 0;
+      const bool has_ac = st.a2 != 0.0;
 #pragma unroll
-      for (int i = 0; i < N1; ++i) y[i] = w[S::ZN + i] + st.a1 * w[S::ZN + N1 + i] + st.a2 * w[S::ACOR + i];
+      for (int i = 0; i < N1; ++i) {
+        const double ac = has_ac ? w[S::ACOR + i] : 0.0;
+        y[i] = w[S::ZN + i] + st.a1 * w[S::ZN + N1 + i] + st.a2 * ac;
+      }
       rhs<M>(y, st.teval, w, st.rE0, st.fH, f, Tsol, &it);
       t_hy2t += (unsigned long long)it;
       if (st.phase == PH_NEWTON) {
         newton = true;
 #pragma unroll
-        for (int i = 0; i < N1; ++i) stage[lane * N1 + i] = st.gamma * f[i] - st.rl1 * w[S::ZN + N1 + i] - w[S::ACOR + i];
+        for (int i = 0; i < N1; ++i) {
+          const double ac = has_ac ? w[S::ACOR + i] : 0.0;
+          stage[lane * N1 + i] = st.gamma * f[i] - st.rl1 * w[S::ZN + N1 + i] - ac;
+        }
       } else {
 #pragma unroll
         for (int i = 0; i < N1; ++i) w[S::F + i] = f[i];
@@ -2651,7 +2829,7 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(OCC) k_persist(const Rea
     //    region ---------------------------------------------------------------------
     bool fresh = false;
     if (act && st.needs_setup() && !st.setup_pending) {
-      st.setup(y, f, Tsol);
+      st.setup(y, f[N], Tsol, w);
       fresh = st.jcur;
     }
     if (__ballot(fresh) != 0ull) {
@@ -2727,51 +2905,21 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(OCC) k_persist(const Rea
     cells_to_rows<N1>(stage, sslot, a.mat, MS::STRIDE, MS::X);
     __syncthreads();
     if (act) {
-      ++st.nfe;
       ++trips;
-      bool reached = false, proceed = true;
-      if (st.setup_pending) proceed = st.after_setup(sing);
-      if (proceed) {
-        switch (st.phase) {
-          case PH_INIT_F0:
+      typename Lane<M>::Newton nw;
+          st.newton_begin(nw, sing);
+      if (nw.on) {
 #pragma unroll
-            for (int i = 0; i < N1; ++i) st.zn(1, i) = w[S::F + i];
-            st.after_f0();
-            break;
-          case PH_HIN:
-#pragma unroll
-            for (int i = 0; i < N1; ++i) f[i] = w[S::F + i];
-            st.after_hin(f);
-            break;
-          case PH_NEWTON:
-            reached = st.iterate();
-            break;
-          case PH_RESTART_F:
-#pragma unroll
-            for (int i = 0; i < N1; ++i) f[i] = w[S::F + i];
-            st.restart_f(f);
-            break;
-          default:
-            break;
-        }
+        for (int i = 0; i < N1; ++i) st.newton_add(nw, i, stage[lane * N1 + i]);
       }
+      bool finite = true;
+      const bool reached = st.trip_end(a, nw, finite);
       if (reached) {
-        // CV_NORMAL output: interpolate the Nordsieck array back to tout
-        const double sfac = (st.tout - st.tn) / st.h;
-        double yo[N1];
-#pragma unroll
-        for (int i = 0; i < N1; ++i) yo[i] = st.zn(st.q, i);
-        for (int j = st.q - 1; j >= 0; --j)
-#pragma unroll
-          for (int i = 0; i < N1; ++i) yo[i] = st.zn(j, i) + sfac * yo[i];
-        bool finite = true;
-#pragma unroll
-        for (int i = 0; i < N1; ++i) finite = finite && isfinite(yo[i]);
         st.finish(finite ? ST_OK : ST_NONFINITE);
         if (finite) {
 #pragma unroll
-          for (int k = 0; k < N; ++k) a.rY.p[cell_off(a.rY, ci, cj, ck) + k * a.rY.ns] = yo[k];
-          a.T.p[cell_off(a.T, ci, cj, ck)] = yo[N];
+          for (int k = 0; k < N; ++k) a.rY.p[cell_off(a.rY, ci, cj, ck) + k * a.rY.ns] = st.zn(0, k);
+          a.T.p[cell_off(a.T, ci, cj, ck)] = st.zn(0, N);
           a.rE.p[cell_off(a.rE, ci, cj, ck)] = st.rE0 + st.fH * st.tout;
         }
       }
@@ -3605,6 +3753,8 @@ hipError_t run_react_t(ReactArgs a, hipStream_t stream, long max_trips, long* tr
   const long n = a.ncell;
   if (a.use_pred && (!pred || !a.compact || !a.plist)) return hipErrorInvalidValue;
   const bool graph = plan.graph_trips > 0 && !prof && !a.use_pred;
+  // the cooperative factorisation in FP64 also solves a set-up's first Newton system
+  a.fuse = (!a.lu_lane && !a.lu_mfma && !a.gmres && a.lu_mode == LU_FP64 && M::N1 <= COOP_MAX_N1) ? 1 : 0;
   Timer* tmp = new Timer();
   tmp->prof = prof;
   tmp->stream = stream;

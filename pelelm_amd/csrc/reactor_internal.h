@@ -50,6 +50,8 @@ struct ReactArgs {
                                          // per wave, blocked; the solves stay cooperative)
   int lu_lane;                           // 1: one lane factors a cell (the form that runs when
                                          // the kernels execute serially on a CPU); 0: 32 lanes
+  int fuse;                              // 1: the factorisation also solves its cell's first Newton
+                                         // system (such cells are not in nlist)
   int gmres;                             // 1: cvode.solve_type = GMRES (no matrix: the Newton
                                          // systems by scaled GMRES with difference-quotient J v)
   int gmres_maxl;                        // its Krylov dimension (1 .. N1 - 1)
