@@ -45,12 +45,22 @@
 #ifndef PELE_SETUP_WAVES
 #define PELE_SETUP_WAVES(N1) ((N1) <= 32 ? 2 : 1)
 #endif
-// k_eval: one wave per SIMD (256 VGPRs plus the accumulation registers, which take the
-// spills) except for the smallest mechanisms, whose right-hand side fits in 128
-// registers; measured on drm19 (spill-free at one wave: 76 -> 68 ms on 128^3) and the
-// 53-species mechanism
+// k_eval: four waves per SIMD where the right-hand side fits in 128 registers, two up to
+// 32 unknowns (drm19 128^3: 33.5 ms; one wave, spill-free, 41; three, with 221 words
+// spilled, 48), one above (the whole register file, the accumulation registers included)
 #ifndef PELE_EVAL_WAVES
-#define PELE_EVAL_WAVES(N1) ((N1) <= 16 ? 4 : 1)
+#define PELE_EVAL_WAVES(N1) ((N1) <= 16 ? 4 : (N1) <= 32 ? 2 : 1)
+#endif
+// the rates kernel (one right-hand side, no integrator state): the same
+// split, measured on the rates of drm19 128^3 (0.51 ms at two waves; four waves, 180
+// words spilled, 0.8)
+#ifndef PELE_RATES_WAVES
+#define PELE_RATES_WAVES(N1) ((N1) <= 16 ? 4 : 2)
+#endif
+// the matrix-free solve: one wave per SIMD above the smallest mechanisms (drm19 16^3: 6.0
+// ms per call, at two waves 7.7)
+#ifndef PELE_GMRES_WAVES
+#define PELE_GMRES_WAVES(N1) ((N1) <= 16 ? 4 : 1)
 #endif
 #ifndef PELE_WAVES_PER_EU
 #define PELE_WAVES_PER_EU(n) __attribute__((amdgpu_waves_per_eu(n)))
@@ -75,6 +85,15 @@
 #else
 #define PELE_HAVE_DODECANE56 1
 #define PELE_HAVE_HEPTANE88 1
+#endif
+// a value that is the same in the wave's active lanes, in a scalar register
+#if defined(__HIP_DEVICE_COMPILE__)
+#define PELE_UNIFORM(x) __builtin_amdgcn_readfirstlane(x)
+#else
+#define PELE_UNIFORM(x) (x)
+#endif
+#ifndef __constant__   // host builds: the generated tables are plain arrays
+#define __constant__
 #endif
 #if defined(PELE_TU_MECH)
 #include PELE_TU_MECH_INC
@@ -209,23 +228,36 @@ __device__ __forceinline__ long cell_off(const IntView& v, int i, int j, int k) 
 // ---------------------------------------------------------------------------
 // right-hand side: T from (rho h)(t) by Newton, then rates and the energy equation
 // ---------------------------------------------------------------------------
+// h and cp of a mixture with NASA coefficients A (M::mix), over R
+__device__ __forceinline__ double mix_h(const double* A, const double T) {
+  return A[5] + T * (A[0] + T * (0.5 * A[1] + T * ((1.0 / 3.0) * A[2] + T * (0.25 * A[3] + T * (0.2 * A[4])))));
+}
+__device__ __forceinline__ double mix_cp(const double* A, const double T) {
+  return A[0] + T * (A[1] + T * (A[2] + T * (A[3] + T * A[4])));
+}
+
+// T from the enthalpy h = sum_k w_k h_k(T), by Newton from T: w mass fractions and h per
+// mass, or w partial densities and h per volume.  A is the mixture's coefficients at the
+// returned T.  The species are summed once per NASA range, not once per iteration: six
+// FMAs each, where evaluating every species' cp and h took an iteration 30 instructions
+// per species.
 template <class M>
-__device__ __forceinline__ double hy2t(const double h, const double* Y, double T, int* iters = nullptr) {
-  double cpR[M::NS], hRT[M::NS];
+__device__ __forceinline__ double hy2t(const double h, const double* w, double T, double* A, int* iters = nullptr) {
+  unsigned range = ~0u;
+  bool found = false;
   int it = 0;
-  for (; it < HY2T_MAXIT; ++it) {
-    M::thermo_cph(T, cpR, hRT);
-    double hT = 0.0, cp = 0.0;
-#pragma unroll
-    for (int k = 0; k < M::NS; ++k) {
-      hT += Y[k] * hRT[k] * M::imw(k);
-      cp += Y[k] * cpR[k] * M::imw(k);
+#pragma unroll 1
+  for (;;) {
+    const unsigned r = M::range(T);
+    if (r != range) {
+      range = r;
+      M::mix(r, w, A);
     }
-    hT *= M::RU * T;
-    cp *= M::RU;
-    const double dT = (h - hT) / cp;
+    if (found || it == HY2T_MAXIT) break;
+    const double dT = (h - M::RU * mix_h(A, T)) / (M::RU * mix_cp(A, T));
     T += dT;
-    if (fabs(dT) <= HY2T_RTOL * T) { ++it; break; }
+    ++it;
+    found = fabs(dT) <= HY2T_RTOL * T;
   }
   if (iters) *iters = it;
   return T;
@@ -236,34 +268,22 @@ __device__ __forceinline__ void rhs(const double* __restrict__ y, const double t
                                     const double fH, double* __restrict__ f, double& Tsol, int* hy2t_iters = nullptr) {
   constexpr int N = M::NS;
   using S = Slots<M::N1>;
-  double rho = 0.0;
-#pragma unroll
-  for (int k = 0; k < N; ++k) rho += y[k];
-  const double irho = 1.0 / rho;
-  double Y[N];
-#pragma unroll
-  for (int k = 0; k < N; ++k) Y[k] = y[k] * irho;
-  const double T = hy2t<M>((rE0 + fH * t) * irho, Y, y[N], hy2t_iters);
+  double A[6];
+  const double T = hy2t<M>(rE0 + fH * t, y, y[N], A, hy2t_iters);   // per volume: rho h of rhoY
   Tsol = T;
+  const double rhocp = M::RU * mix_cp(A, T);
   const double logT = log(T), invT = 1.0 / T;
   double C[N], g[N], wd[N];
 #pragma unroll
   for (int k = 0; k < N; ++k) C[k] = y[k] * M::imw(k);
   M::gibbs(T, logT, g);
   M::wdot(C, T, logT, invT, g, wd);
-  double cpR[N], hRT[N];
-  M::thermo_cph(T, cpR, hRT);
+#pragma unroll
+  for (int k = 0; k < N; ++k) f[k] = wd[k] * M::mw(k) + ws[S::FY + k];
   // energy closure from rho h = sum_k rhoY_k h_k(T): rho cp dT/dt = F_h - sum_k h_k d(rhoY_k)/dt
   // with d(rhoY_k)/dt = W_k wdot_k + F_Y,k (the species forcing carries its enthalpy)
-  double rhocp = 0.0, hw = 0.0;
-#pragma unroll
-  for (int k = 0; k < N; ++k) {
-    const double fy = ws[S::FY + k];
-    f[k] = wd[k] * M::mw(k) + fy;
-    rhocp += y[k] * cpR[k] * M::imw(k);
-    hw += (wd[k] + fy * M::imw(k)) * hRT[k];
-  }
-  f[N] = (fH - hw * M::RU * T) / (rhocp * M::RU);
+  M::mix(M::range(T), f, A);
+  f[N] = (fH - M::RU * mix_h(A, T)) / rhocp;
 }
 
 // analytic Jacobian of the right-hand side at (y, T) with T held fixed, into js[JS] (the
@@ -2481,7 +2501,7 @@ __device__ __forceinline__ int gmres_cell(const WS& w, const CM& mat, const HS& 
 // (MatSlots IRF) tells the step kernel whether the linear solve failed, IRS holds its
 // Krylov iterations
 template <class M>
-__global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(PELE_EVAL_WAVES(M::N1)) k_solve_gmres(
+__global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(PELE_GMRES_WAVES(M::N1)) k_solve_gmres(
     const ReactArgs a, const int* __restrict__ list, const unsigned int* __restrict__ count) {
   using MS = MatSlots<M::N1>;
   __shared__ double sg[GMRES_LDS_WORDS * 64];
@@ -2968,13 +2988,14 @@ __global__ void k_plain_counts(unsigned int* counts, unsigned int n) {
 
 // net production rates rho*wdot (g/cm^3/s) with T re-solved from h
 // reactionRateRhoY per cell (Source/PeleLM_K.H:57-98): rho = sum_k rhoY_k, Y = rhoY / rho,
-// h = rhoH / rho x hscale, T = HY2T(h, Y) started from the T the cell holds (T itself is
+// h = rhoH / rho x hscale (solved per volume, so that rho drops out), T = HY2T(h, Y)
+// started from the T the cell holds (T itself is
 // read only; the re-solved value goes to Tout when given), and
 // rhoYdot_k = W_k wdot_k(rho x rscale, T, Y) x oscale.  The box form passes PeleLM's MKS
 // factors (hscale 1e4, rscale 1e-3, oscale 1e3), the flat CGS form 1, 1, 1.  Cells with
 // mask < 0 (EB-covered) get zero rates.
 template <class M>
-__global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(4) rates_kernel(const ArrView rhoY, const ArrView rhoH,
+__global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(PELE_RATES_WAVES(M::N1)) rates_kernel(const ArrView rhoY, const ArrView rhoH,
                                                                         const ArrView T, const IntView mask,
                                                                         const ArrView rdot, double* __restrict__ Tout,
                                                                         const int nx, const int ny, const long ncell,
@@ -2991,18 +3012,16 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(4) rates_kernel(const Ar
     return;
   }
   const long oy = cell_off(rhoY, i, j, k);
-  double Y[N], rho = 0.0;
+  double Y[N], A[6];
 #pragma unroll
-  for (int n = 0; n < N; ++n) { Y[n] = rhoY.p[oy + n * rhoY.ns]; rho += Y[n]; }
-  const double irho = 1.0 / rho;
-#pragma unroll
-  for (int n = 0; n < N; ++n) Y[n] *= irho;
-  const double Tc = hy2t<M>(rhoH.p[cell_off(rhoH, i, j, k)] * irho * hscale, Y, T.p[cell_off(T, i, j, k)]);
+  for (int n = 0; n < N; ++n) Y[n] = rhoY.p[oy + n * rhoY.ns];
+  // per volume: rho h = sum_k rhoY_k h_k(T)
+  const double Tc = hy2t<M>(rhoH.p[cell_off(rhoH, i, j, k)] * hscale, Y, T.p[cell_off(T, i, j, k)], A);
   if (Tout) Tout[c] = Tc;
-  const double rho_c = rho * rscale, logT = log(Tc), invT = 1.0 / Tc;
+  const double logT = log(Tc), invT = 1.0 / Tc;
   double C[N], g[N], wd[N];
 #pragma unroll
-  for (int n = 0; n < N; ++n) C[n] = rho_c * Y[n] * M::imw(n);
+  for (int n = 0; n < N; ++n) C[n] = rscale * Y[n] * M::imw(n);
   M::gibbs(Tc, logT, g);
   M::wdot(C, Tc, logT, invT, g, wd);
 #pragma unroll
@@ -3019,7 +3038,7 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(4) rates_kernel(const Ar
 //               species changes over dt
 // Cells with mask < 0 get key 0.
 template <class M>
-__global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(4) k_cost_key(const ReactArgs a, const int mode,
+__global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(PELE_EVAL_WAVES(M::N1)) k_cost_key(const ReactArgs a, const int mode,
                                                                       unsigned int* __restrict__ keys,
                                                                       int* __restrict__ vals) {
   constexpr int N = M::NS;
@@ -3034,13 +3053,10 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(4) k_cost_key(const Reac
     key = isfinite(fc) ? (float)fmin(fc, 3.0e38) : 3.0e38f;
   } else if (!masked && mode == ORDER_RATE) {
     const long oy = cell_off(a.rY, i, j, k);
-    double y[N], Y[N], rho = 0.0;
+    double y[N], A[6];
 #pragma unroll
-    for (int n = 0; n < N; ++n) { y[n] = a.rY.p[oy + n * a.rY.ns]; rho += y[n]; }
-    const double irho = 1.0 / rho;
-#pragma unroll
-    for (int n = 0; n < N; ++n) Y[n] = y[n] * irho;
-    const double T = hy2t<M>(a.rE.p[cell_off(a.rE, i, j, k)] * irho, Y, a.T.p[cell_off(a.T, i, j, k)]);
+    for (int n = 0; n < N; ++n) y[n] = a.rY.p[oy + n * a.rY.ns];
+    const double T = hy2t<M>(a.rE.p[cell_off(a.rE, i, j, k)], y, a.T.p[cell_off(a.T, i, j, k)], A);
     const double logT = log(T), invT = 1.0 / T;
     double C[N], g[N], wd[N];
 #pragma unroll
@@ -3931,7 +3947,8 @@ __global__ void __launch_bounds__(64) rhoh_to_temp_kernel(const ArrView rho, con
   for (int n = 0; n < N; ++n) y[n] = rhoY.p[oy + n * rhoY.ns] * rhoinv;
   const double h_cgs = rhoH.p[cell_off(rhoH, i, j, k)] * rhoinv * 1.0e4;
   const long ot = cell_off(T, i, j, k);
-  T.p[ot] = hy2t<M>(h_cgs, y, T.p[ot]);
+  double A[6];
+  T.p[ot] = hy2t<M>(h_cgs, y, T.p[ot], A);
 }
 
 template <class M>

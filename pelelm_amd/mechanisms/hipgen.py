@@ -1,20 +1,36 @@
-"""Emit straight-line HIP device code for one mechanism (one cell per lane).
+"""Emit HIP device code for one mechanism (one cell per lane).
 
 The generated header defines ``struct mech_<name>`` with static members:
 
 * ``NS``, ``NR``, ``N1`` and the constant tables host code needs (molecular weights,
-  NASA-7 coefficients, species names);
-* ``thermo_cph(T, cpR, hRT)`` -- cp/R and h/RT of every species (HY2T, energy equation);
-* ``gibbs(T, logT, gRT)`` -- g/RT;
+  species names);
+* ``range(T)`` and ``mix(range, w, A)`` -- the NASA-7 range of a temperature, and the
+  mixture's coefficients A_j = sum_k w_k a_jk / W_k in it, so that h and cp of a mixture
+  are one polynomial each (HY2T, energy equation);
+* ``thermo_cph(T, cpR, hRT)``, ``thermo_dcp(T, dcpR)`` -- cp/R, h/RT and d(cp/R)/dT of
+  every species (Jacobian);
+* ``gibbs(T, logT, gRT)`` -- g/RT, each element's potential shifted by a constant that no
+  balanced reaction sees (``_element_shift``);
 * ``wdot(C, T, logT, invT, gRT, wd)`` -- net molar production rates [mol/cm^3/s];
 * ``jacobian(C, T, logT, invT, gRT, hRT, wd, dwdT, acc)`` -- the analytic derivatives
   d(wdot_i W_i)/d(rhoY_k) accumulated through ``acc(i, k, value)`` plus dwdot/dT.
 
-NASA-7 range selection is branch-free (coefficients chosen with a select on
-T < Tmid) so lanes on both sides of the break temperature stay converged.  Constant
-folding: k_f with beta = Ea = 0 is a literal; Troe terms with T*** = 1e-30 / T* = 1e30
-vanish / become constants; third-body sums start from the total concentration and
-add (eff - 1) C_k only for species with non-unit efficiency.
+The NASA-7 coefficients come from tables in constant memory whose address is uniform over
+a wave (scalar loads, one scalar operand per FMA): the two ranges are the two trips of a
+loop that a wave enters for the lanes on that side, so a wave on one side runs one of
+them.  (Coefficients written as selects between two literals cost four moves and two
+selects each, three times the polynomial's own arithmetic.)
+
+Every transcendental of a state is evaluated once: exp(g_k/RT) and its reciprocal per
+species instead of exp(-dG/RT) per reaction, and exp(b ln T - Ta/T) once per distinct
+(b, Ta), the reactions that share it emitted next to each other.  drm19: 199 of them
+become 133; the 88-species mechanism: 856 become 278.  Troe terms with T*** = 1e-30 /
+T* = 1e30 vanish / become constants; third-body sums start from the total concentration
+and add (eff - 1) C_k only for species with non-unit efficiency.
+
+``gen_thermo``, ``gen_wdot`` and ``gen_jacobian(shared=False)`` write the same arithmetic
+out species by species and reaction by reaction; the operation counts are counted on that
+form, which says what a mechanism asks for and not how the emitted code saves on it.
 """
 from __future__ import annotations
 
@@ -22,6 +38,8 @@ import json
 import math
 import os
 import re
+
+import numpy as np
 
 from . import mechanism as M
 
@@ -104,6 +122,108 @@ def gen_thermo(mech: M.Mechanism) -> str:
             out.append(f"      gRT[{k}] = a0 * (1.0 - logT) - 0.5 * a1 * T - (1.0 / 6.0) * a2 * T2 - (1.0 / 12.0) * a3 * T3"
                        f" - 0.05 * a4 * T4 + a5 * iT - a6; }}")
         out.append("  }")
+    out.append("}")
+    return "\n".join(out)
+
+
+def _element_shift(mech: M.Mechanism) -> list:
+    """(d5, d6) per species: what to add to the NASA coefficients a5 and a6 so that g/RT
+    loses sum_e n_ke (alpha_e + beta_e / T).  A reaction that conserves its elements does
+    not see it, while exp(g/RT) of every species, and the product over either side of a
+    reaction, stays within the range of a double down to 200 K, as the exponential of the
+    reaction's own difference does.  alpha and beta are the least-squares fit of g/RT over
+    200 - 4000 K, rounded (1, and 10 K)."""
+    els = list(mech.elements)
+    for r in mech.reactions:
+        for e in els:
+            n = sum(c * mech.species[i].composition.get(e, 0) for i, c in r.products.items()) - \
+                sum(c * mech.species[i].composition.get(e, 0) for i, c in r.reactants.items())
+            if n != 0:
+                return [(0.0, 0.0)] * mech.nspec
+    rows, rhs = [], []
+    for s in mech.species:
+        for T in (200.0, 250.0, 300.0, 400.0, 600.0, 1000.0, 1500.0, 2500.0, 4000.0):
+            a = s.low if T < s.T[1] else s.high
+            n = [s.composition.get(e, 0) for e in els]
+            rows.append(n + [x * 1000.0 / T for x in n])
+            rhs.append(a[0] * (1.0 - math.log(T)) - a[1] * T / 2 - a[2] * T ** 2 / 6 - a[3] * T ** 3 / 12
+                       - a[4] * T ** 4 / 20 + a[5] / T - a[6])
+    x = np.linalg.lstsq(np.array(rows), np.array(rhs), rcond=None)[0]
+    alpha = [float(round(v)) for v in x[:len(els)]]
+    beta = [10.0 * round(100.0 * v) for v in x[len(els):]]
+    return [(-sum(b * s.composition.get(e, 0) for e, b in zip(els, beta)),
+             sum(v * s.composition.get(e, 0) for e, v in zip(els, alpha))) for s in mech.species]
+
+
+def gen_tables(mech: M.Mechanism) -> str:
+    """The constant-memory tables, [range][species][8]: NASA coefficients over the
+    molecular weight (mixture sums), as they are (per species), and g/RT's (a0, a1/2,
+    a2/6, a3/12, a4/20, a5, a6, shifted)."""
+    cn = _cname(mech.name)
+    shift = _element_shift(mech)
+    out = []
+
+    def table(name, row):
+        out.append(f"static __constant__ double {cn}_{name}[2][{mech.nspec}][8] = {{")
+        for side in (0, 1):
+            out.append(" {")
+            for k, s in enumerate(mech.species):
+                out.append("  {" + ", ".join(_d(v) for v in row(k, s, s.low if side == 0 else s.high)) + "},")
+            out.append(" },")
+        out.append("};")
+
+    table("mass", lambda k, s, a: [a[i] / mech.W[k] for i in range(6)] + [0.0, 0.0])
+    table("nasa", lambda k, s, a: [a[i] for i in range(7)] + [0.0])
+    table("gibbs", lambda k, s, a: [a[0], a[1] / 2.0, a[2] / 6.0, a[3] / 12.0, a[4] / 20.0, a[5] + shift[k][0],
+                                    a[6] + shift[k][1], 0.0])
+    return "\n".join(out)
+
+
+def gen_thermo_tables(mech: M.Mechanism) -> str:
+    cn = _cname(mech.name)
+    groups = list(_thermo_groups(mech).items())
+    out = []
+
+    def sided(body):
+        # body(k) for every species, u naming its table's range
+        for g, (tmid, ks) in enumerate(groups):
+            out.append("#pragma unroll 1")
+            out.append(f"  for (int r = 0; r < 2; ++r) if ((int)((range >> {g}) & 1u) == r) {{")
+            # inside the branch the compiler knows r to be the lane's own bit: keep it scalar
+            out.append("    const int u = PELE_UNIFORM(r);")
+            for k in ks:
+                out.append("    " + body(k))
+            out.append("  }")
+
+    out.append("// one bit per break temperature: T in its upper range")
+    out.append("static __device__ __forceinline__ unsigned range(const double T) {")
+    out.append("  return " + " | ".join(f"(T < {_d(t)} ? 0u : {1 << g}u)" for g, (t, _) in enumerate(groups)) + ";")
+    out.append("}")
+    out.append("// A[j] = sum_k w_k a_jk / W_k, j = 0..5")
+    out.append("static __device__ __forceinline__ void mix(const unsigned range, const double* __restrict__ w, "
+               "double* __restrict__ A) {")
+    out.append("  for (int j = 0; j < 6; ++j) A[j] = 0.0;")
+    sided(lambda k: f"{{ const double* t = {cn}_mass[u][{k}]; for (int j = 0; j < 6; ++j) A[j] += w[{k}] * t[j]; }}")
+    out.append("}")
+    out.append("static __device__ __forceinline__ void thermo_cph(const double T, double* __restrict__ cpR, "
+               "double* __restrict__ hRT) {")
+    out.append("  const double iT = 1.0 / T;")
+    out.append("  const unsigned range = mech_" + cn + "::range(T);")
+    sided(lambda k: f"{{ const double* t = {cn}_nasa[u][{k}];"
+                    f" cpR[{k}] = t[0] + T * (t[1] + T * (t[2] + T * (t[3] + T * t[4])));"
+                    f" hRT[{k}] = t[0] + T * (0.5 * t[1] + T * ((1.0 / 3.0) * t[2] + T * (0.25 * t[3] + T * (0.2 * t[4]))))"
+                    f" + t[5] * iT; }}")
+    out.append("}")
+    out.append("static __device__ __forceinline__ void thermo_dcp(const double T, double* __restrict__ dcpR) {")
+    out.append("  const unsigned range = mech_" + cn + "::range(T);")
+    sided(lambda k: f"{{ const double* t = {cn}_nasa[u][{k}];"
+                    f" dcpR[{k}] = t[1] + T * (2.0 * t[2] + T * (3.0 * t[3] + T * (4.0 * t[4]))); }}")
+    out.append("}")
+    out.append("static __device__ __forceinline__ void gibbs(const double T, const double logT, double* __restrict__ gRT) {")
+    out.append("  const double iT = 1.0 / T, l1 = 1.0 - logT;")
+    out.append("  const unsigned range = mech_" + cn + "::range(T);")
+    sided(lambda k: f"{{ const double* t = {cn}_gibbs[u][{k}];"
+                    f" gRT[{k}] = t[0] * l1 - T * (t[1] + T * (t[2] + T * (t[3] + T * t[4]))) + t[5] * iT - t[6]; }}")
     out.append("}")
     return "\n".join(out)
 
@@ -231,7 +351,93 @@ def gen_wdot(mech: M.Mechanism) -> str:
     return "\n".join(out)
 
 
-def gen_jacobian(mech: M.Mechanism) -> str:
+def _exponent(b: float, Ta: float) -> str:
+    return " + ".join(([f"{_d(b)} * logT"] if b != 0.0 else []) + ([f"{_d(-Ta)} * invT"] if Ta != 0.0 else []))
+
+
+def _rate_groups(mech: M.Mechanism) -> list:
+    """Reactions grouped by the (b, Ta) of their rate constant, third-body ones first
+    (they read the concentrations, the others only C exp(g/RT)); the group (0, 0) needs no
+    exponential."""
+    groups: dict = {}
+    for j, r in enumerate(mech.reactions):
+        groups.setdefault((not r.has_third_body, r.beta, r.Ea), []).append(j)
+    return sorted(((k[1], k[2], js) for k, js in groups.items()),
+                  key=lambda g: (not mech.reactions[g[2][0]].has_third_body, g[2][0]))
+
+
+def _species_exps(mech: M.Mechanism) -> list:
+    return ["  double E[NS], I[NS];   // exp(g/RT) and its reciprocal",
+            "#pragma unroll",
+            "  for (int k = 0; k < NS; ++k) { E[k] = exp(gRT[k]); I[k] = 1.0 / E[k]; }"]
+
+
+def gen_wdot_shared(mech: M.Mechanism) -> str:
+    """The production rates with every transcendental evaluated once.  With X_k = C_k
+    exp(g_k/RT), a reaction's net rate is kf prod_f exp(-g/RT) (prod_f X - prod_r X
+    (P_atm/RT)^-dnu)."""
+    ns = mech.nspec
+    out = []
+    out.append("static __device__ __forceinline__ void wdot(const double* __restrict__ C, const double T, const double logT, "
+               "const double invT, const double* __restrict__ gRT, double* __restrict__ wd) {")
+    out.append(f"  const double refC = {_d(M.P_ATM / M.R_CGS)} * invT, refCinv = 1.0 / refC;")
+    out += _species_exps(mech)
+    out.append("  double X[NS];")
+    out.append("#pragma unroll")
+    out.append("  for (int k = 0; k < NS; ++k) { X[k] = C[k] * E[k]; wd[k] = 0.0; }")
+    if any(r.has_third_body for r in mech.reactions):
+        out.append("  double Ctot = 0.0;")
+        out.append("#pragma unroll")
+        out.append("  for (int k = 0; k < NS; ++k) Ctot += C[k];")
+
+    def xs(side):
+        return _prod([t for i, c in sorted(side.items()) for t in [f"X[{i}]"] * c])
+
+    for b, Ea, js in _rate_groups(mech):
+        x = _exponent(b, Ea / M.R_CAL)
+        if x:
+            out.append(f"  {{ const double x = exp({x});")
+        else:
+            out.append("  {")
+        for j in js:
+            r = mech.reactions[j]
+            out.append(f"  {{ // {j}: {r.equation}")
+            out.append(f"    const double kf = {_d(r.A)}{' * x' if x else ''};")
+            if r.kind == "elementary":
+                out.append("    const double keff = kf;")
+            elif r.kind == "three-body":
+                out.append(f"    const double keff = kf * ({_mc_expr(r, ns)});")
+            else:
+                A0, b0, E0 = r.low
+                out.append(f"    const double k0 = {_kf_expr(A0, b0, E0 / M.R_CAL)};")
+                out.append(f"    const double Pr = k0 * ({_mc_expr(r, ns)}) / kf;")
+                if r.troe is not None:
+                    fc, _ = _troe_fc(r)
+                    out.append(f"    const double logFc = log10(fmax({fc}, 1e-300));")
+                    out.append("    const double cc = -0.4 - 0.67 * logFc, nn = 0.75 - 1.27 * logFc;")
+                    out.append("    const double u = log10(fmax(Pr, 1e-300)) + cc;")
+                    out.append("    const double f1 = u / (nn - 0.14 * u);")
+                    out.append("    const double F = exp(2.302585092994045684 * logFc / (1.0 + f1 * f1));")
+                    out.append("    const double keff = kf * Pr / (1.0 + Pr) * F;")
+                else:
+                    out.append("    const double keff = kf * Pr / (1.0 + Pr);")
+            back = ""
+            if r.reversible:
+                dnu = sum(r.products.values()) - sum(r.reactants.values())
+                back = f" - {xs(r.products)}{_refc_factor(dnu)}"
+            inv = "".join(f" * I[{i}]" * c for i, c in sorted(r.reactants.items()))
+            out.append(f"    const double q = keff{inv} * ({xs(r.reactants)}{back});")
+            for i, c in sorted(r.reactants.items()):
+                out.append(f"    wd[{i}] -= {_d(c) + ' * ' if c != 1 else ''}q;")
+            for i, c in sorted(r.products.items()):
+                out.append(f"    wd[{i}] += {_d(c) + ' * ' if c != 1 else ''}q;")
+            out.append("  }")
+        out.append("  }")
+    out.append("}")
+    return "\n".join(out)
+
+
+def gen_jacobian(mech: M.Mechanism, shared: bool = True) -> str:
     """Derivatives of f_i = W_i wdot_i with respect to rhoY_k (=W_k C_k) and T.
 
     Two phases, so that no Jacobian entry is accumulated in memory (a read-modify-
@@ -241,7 +447,8 @@ def gen_jacobian(mech: M.Mechanism) -> str:
     ascending, rows i ascending, structural zeros included), each sum over reactions in
     reaction order.  acc(i, k, v) receives each entry v = sum_j W_i/W_k nu_ij dq_j/dC_k
     exactly once, and colend(k) follows the last row of column k.  dwdT is the molar
-    dwdot/dT and wd the molar production rates at the same state.
+    dwdot/dT and wd the molar production rates at the same state.  shared: with every
+    transcendental evaluated once, as in ``gen_wdot_shared``.
     """
     ns = mech.nspec
     nr = mech.nreac
@@ -254,9 +461,17 @@ def gen_jacobian(mech: M.Mechanism) -> str:
     if any(r.has_third_body for r in mech.reactions):
         body.append("  double Ctot = 0.0;")
         body.append(f"  for (int k = 0; k < {ns}; ++k) Ctot += C[k];")
+    blocks = []          # per reaction: its lines
     for j, r in enumerate(mech.reactions):
+        head, body = body, []
+        blocks.append(body)
+        if j == 0:
+            first = head
         body.append(f"  {{ // {j}: {r.equation}")
-        body.append(f"    const double kf = {_kf_expr(r.A, r.beta, r.Ea / M.R_CAL)};")
+        if shared:
+            body.append(f"    const double kf = {_d(r.A)}{' * x' if r.beta != 0.0 or r.Ea != 0.0 else ''};")
+        else:
+            body.append(f"    const double kf = {_kf_expr(r.A, r.beta, r.Ea / M.R_CAL)};")
         body.append(f"    const double dlnkf = {_dlnk_expr(r.beta, r.Ea / M.R_CAL)};")
         if r.kind == "elementary":
             body.append("    const double keff = kf, dkeffdT = kf * dlnkf;")
@@ -294,7 +509,12 @@ def gen_jacobian(mech: M.Mechanism) -> str:
             gs, hs, dnu = _kc_exprs(r)
             pr = _prod(_power_terms(r.products))
             body.append(f"    const double pr = {pr};")
-            body.append(f"    const double invKc = exp({gs}){_refc_factor(dnu)};")
+            if shared:
+                gs = " * ".join([f"E[{i}]" for i, c in sorted(r.products.items()) for _ in range(c)]
+                                + [f"I[{i}]" for i, c in sorted(r.reactants.items()) for _ in range(c)])
+                body.append(f"    const double invKc = {gs}{_refc_factor(dnu)};")
+            else:
+                body.append(f"    const double invKc = exp({gs}){_refc_factor(dnu)};")
             body.append(f"    const double dlnKc = ({hs} - {_d(dnu)}) * invT;")
             body.append("    const double net = pf - pr * invKc;")
             body.append("    const double dqdT = dkeffdT * net + keff * pr * invKc * dlnKc;")
@@ -339,7 +559,19 @@ def gen_jacobian(mech: M.Mechanism) -> str:
                "double* __restrict__ wd, double* __restrict__ dwdT, Acc&& acc, ColEnd&& colend) {")
     out.append(f"  const double refC = {_d(M.P_ATM / M.R_CGS)} * invT, refCinv = 1.0 / refC;")
     out.append(f"  double Q[{nr}], QT[{nr}], D[{max(nd, 1)}];")
-    out += body
+    if not shared:
+        out += first
+        for b in blocks:
+            out += b
+    else:
+        out += _species_exps(mech)
+        out += first
+        for b, Ea, js in _rate_groups(mech):
+            x = _exponent(b, Ea / M.R_CAL)
+            out.append(f"  {{ const double x = exp({x});" if x else "  {")
+            for j in js:
+                out += blocks[j]
+            out.append("  }")
     # production rates and their T derivatives, species by species
     for i in range(ns):
         terms = [(nu_all[j][i], j) for j in range(nr) if i in nu_all[j]]
@@ -408,6 +640,7 @@ def write_inc(mech: M.Mechanism, path: str) -> None:
     cn = _cname(name)
     lines = [f"// GENERATED by pelelm_amd/mechanisms/hipgen.py from {name}.yaml -- do not edit.",
              f"// {ns} species, {mech.nreac} reactions.", "#pragma once", "",
+             gen_tables(mech), "",
              f"struct mech_{cn} {{", "",
              f"static constexpr int NS = {ns};", f"static constexpr int NR = {mech.nreac};",
              f"static constexpr int N1 = {ns + 1};",
@@ -425,7 +658,7 @@ def write_inc(mech: M.Mechanism, path: str) -> None:
              ""]
     th = gen_thermo(mech)
     wd = gen_wdot(mech)
-    jac = gen_jacobian(mech)
+    jac = gen_jacobian(mech, shared=False)
     parts = th.split("static __device__ __forceinline__ void ")
     counts = {}
     for part in parts[1:]:
@@ -433,16 +666,17 @@ def write_inc(mech: M.Mechanism, path: str) -> None:
         counts[fname] = count_ops(part)
     counts["wdot"] = count_ops(wd)
     counts["jacobian"] = count_ops(jac)
-    lines.append("// static operation counts (flops; transcendentals) of the generated functions")
+    lines.append("// static operation counts (flops; transcendentals) of the functions, written out species by")
+    lines.append("// species and reaction by reaction")
     for k, v in counts.items():
         lines.append(f"static constexpr long OPS_{k.upper()} = {v['flops']};")
         lines.append(f"static constexpr long TRANS_{k.upper()} = {v['transcendentals']};")
     lines.append("")
-    lines.append(th)
+    lines.append(gen_thermo_tables(mech))
     lines.append("")
-    lines.append(wd)
+    lines.append(gen_wdot_shared(mech))
     lines.append("")
-    lines.append(jac)
+    lines.append(gen_jacobian(mech))
     lines.append("")
     lines.append(f"}};  // struct mech_{cn}")
     with open(path, "w") as f:
