@@ -108,6 +108,9 @@ struct Reactor {
   unsigned long long* stat_counters = nullptr;
   long last_trips = 0;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  // a trip's counts on their way to the host (TripPlan)
+  unsigned int* host_counts = nullptr;
+  hipEvent_t counted = nullptr;
   hipStream_t last_stream = nullptr;
   bool have_stats = false;
   long last_ncell = 0;
@@ -146,6 +149,10 @@ int ensure_device_state(Reactor* r, long ncell) {
     HIPCHK(r, hipMalloc(&r->counters, NCOUNTERS * sizeof(unsigned long long)));
     if (!r->ev0) HIPCHK(r, hipEventCreate(&r->ev0));
     if (!r->ev1) HIPCHK(r, hipEventCreate(&r->ev1));
+    if (hipHostMalloc(reinterpret_cast<void**>(&r->host_counts), 8 * sizeof(unsigned int), hipHostMallocDefault) !=
+        hipSuccess)
+      return fail(r, MI_ENOMEM, "pinned host memory: allocation failed");
+    HIPCHK(r, hipEventCreateWithFlags(&r->counted, hipEventDisableTiming));
   }
   if (ncell > r->ws_cells) {
     free_workspace(r);
@@ -448,6 +455,8 @@ int trial(Reactor* r, ReactArgs a, const TuneConfig& c, hipStream_t stream, long
     TripPlan plan;
     plan.graph_trips = c.graph_trips;
     plan.capture_stream = r->capture_stream;
+    plan.host_counts = r->host_counts;
+    plan.counted = r->counted;
     long trips = 0;
     HIPCHK(r, run_react(r->mech, a, stream, max_trips, &trips, nullptr, nullptr, plan));
   }
@@ -680,6 +689,8 @@ int react_common(Reactor* r, ReactArgs& a, double* dt, double* time, hipStream_t
     TripPlan plan;
     plan.graph_trips = graph_trips;
     plan.capture_stream = r->capture_stream;
+    plan.host_counts = r->host_counts;
+    plan.counted = r->counted;
     HIPCHK(r, run_react(r->mech, a, stream, max_trips, &r->last_trips, r->profile ? &r->prof : nullptr,
                         mlp_device(r->predictor), plan));
   }
@@ -1249,6 +1260,8 @@ int mi_chem_close(void* reactor) {
   if (r->counters) (void)hipFree(r->counters);
   if (r->ev0) (void)hipEventDestroy(r->ev0);
   if (r->ev1) (void)hipEventDestroy(r->ev1);
+  if (r->host_counts) (void)hipHostFree(r->host_counts);
+  if (r->counted) (void)hipEventDestroy(r->counted);
   if (r->capture_stream) (void)hipStreamDestroy(r->capture_stream);
   delete r;
   return MI_OK;

@@ -2979,6 +2979,16 @@ __global__ void k_zero_two(unsigned int* counts, int i0, int i1) {
     counts[i1] = 0u;
   }
 }
+// start of a trip: clear the lists it fills (and the solve list's count); with `tally`,
+// count it in counts[7] if any cell is still integrating (counts[act])
+__global__ void k_trip_start(unsigned int* counts, int act, int i0, int i1, int tally) {
+  if (threadIdx.x == 0) {
+    if (tally && counts[act] != 0u) ++counts[7];
+    counts[i0] = 0u;
+    counts[i1] = 0u;
+    counts[6] = 0u;
+  }
+}
 __global__ void k_plain_counts(unsigned int* counts, unsigned int n) {
   if (threadIdx.x == 0) {
     counts[4] = n;
@@ -3633,7 +3643,7 @@ hipError_t launch_solve(const ReactArgs& a, long n, hipStream_t stream) {
 // counts[0..1]: active-cell lists of the current / next trip, counts[2..3]: their set-up
 // lists; without compaction counts[4] is the (fixed) list length and counts[5] the
 // number of cells still integrating; counts[6]: cells due a Newton solve this trip;
-// counts[7]: cells awaiting a learned prediction.
+// counts[7]: cells awaiting a learned prediction, or (batched trips) the trips that had work.
 // Per-kernel timing: an event pair per launch, recorded asynchronously and read back
 // once the call has finished, so profiling adds no synchronisation inside the trips.
 struct Timer {
@@ -3689,29 +3699,29 @@ hipError_t launch_predict(const ReactArgs& a, const MlpDev& w, unsigned np, hipS
 }
 
 // One trip with grids sized for every cell (kernels skip beyond their list counts), as
-// captured into a graph: evaluation, set-up, factorisation, solves, step logic.
+// captured into a graph or issued several at a time: evaluation, set-up, factorisation,
+// solves, step logic.  exact: the factorisation's grid covers ncell cells (else a fixed
+// grid strides over them); tally: the trip is counted in counts[7].
 template <class M>
-hipError_t enqueue_fixed_trip(const ReactArgs& a, int cur, hipStream_t s) {
+hipError_t enqueue_fixed_trip(const ReactArgs& a, int cur, hipStream_t s, bool exact = false, int tally = 0) {
   const long n = a.ncell;
   const unsigned nb = (unsigned)((n + 63) / 64);
   const int nxt = 1 - cur;
-  if (a.compact)
-    hipLaunchKernelGGL(k_zero_two, dim3(1), dim3(64), 0, s, a.counts, nxt, 2 + nxt);
-  else
-    hipLaunchKernelGGL(k_zero_two, dim3(1), dim3(64), 0, s, a.counts, 5, 2 + nxt);
-  PELE_TRY(hipGetLastError());
-  hipLaunchKernelGGL(k_zero_two, dim3(1), dim3(64), 0, s, a.counts, 6, 6);
+  hipLaunchKernelGGL(k_trip_start, dim3(1), dim3(64), 0, s, a.counts, a.compact ? cur : 5, a.compact ? nxt : 5, 2 + nxt,
+                     tally);
   PELE_TRY(hipGetLastError());
   const int* act = a.compact ? a.list[cur] : a.list[1];
   const unsigned* act_n = a.compact ? &a.counts[cur] : &a.counts[4];
   hipLaunchKernelGGL(k_eval<M>, dim3(nb), dim3(64), 0, s, a, act, act_n);
   PELE_TRY(hipGetLastError());
-  hipLaunchKernelGGL(k_setup<M>, dim3(nb), dim3(64), 0, s, a, a.slist[cur], &a.counts[2 + cur]);
-  PELE_TRY(hipGetLastError());
-  PELE_TRY(launch_lu<M>(a, a.slist[cur], &a.counts[2 + cur], n, s, false));
+  if (!a.gmres) {
+    hipLaunchKernelGGL(k_setup<M>, dim3(nb), dim3(64), 0, s, a, a.slist[cur], &a.counts[2 + cur]);
+    PELE_TRY(hipGetLastError());
+    PELE_TRY(launch_lu<M>(a, a.slist[cur], &a.counts[2 + cur], n, s, exact));
+  }
   // the cooperative solve strides over its list from a fixed grid; the one-lane solve
   // takes one cell per lane, so its grid covers every cell the list can hold
-  PELE_TRY(launch_solve<M>(a, (a.lu_lane || a.gmres) ? n : 16384, s));
+  PELE_TRY(launch_solve<M>(a, (a.lu_lane || a.gmres || exact) ? n : 16384, s));
   if (a.compact)
     hipLaunchKernelGGL(k_consume<M>, dim3(nb), dim3(64), 0, s, a, act, act_n, a.list[nxt], &a.counts[nxt],
                        a.slist[nxt], &a.counts[2 + nxt]);
@@ -3763,6 +3773,20 @@ hipError_t run_trips_graph(const ReactArgs& a, hipStream_t stream, long max_trip
   return hipSuccess;
 }
 
+// Boxes up to batch_cells cells run BATCH_TRIPS trips between two looks at the device's
+// counts, with grids for every cell; above, each trip's grids fit its lists.  A look costs
+// 35 us of idle GPU per trip, a third of a trip on a LiDryer 16^3 box (5.5 -> 4.0 ms per
+// call; drm19 16^3 with GMRES 9.3 -> 8.8, 17x15x13 with forcing 10.6 -> 10.0); a trip after
+// the last cell has finished, 25 us of empty kernels.  The line lies where a factorisation
+// grid's empty blocks cost less than the look: 10 ns a block of one wave (56 species,
+// 29,667 blocks: 0.3 ms a trip, a call 101 -> 157 ms), 46 of two waves (88 species, 32,768
+// blocks: 446 -> 709 ms); two cells share a block up to 32 unknowns.
+template <int N1>
+constexpr long batch_cells() {
+  return N1 <= 32 ? 4096 : N1 <= 64 ? 2048 : 512;
+}
+constexpr int BATCH_TRIPS = 8;
+
 template <class M>
 hipError_t run_react_t(ReactArgs a, hipStream_t stream, long max_trips, long* trips_out, KernelProf* prof,
                        const MlpDev* pred, const TripPlan& plan) {
@@ -3794,17 +3818,46 @@ hipError_t run_react_t(ReactArgs a, hipStream_t stream, long max_trips, long* tr
   int cur = 0;
   long trip = 0;
   unsigned int h_counts[8];
-  for (; trip < max_trips; ++trip) {
+  // small boxes: several trips per look at the counts (not while profiling, which wants
+  // each launch's cells, nor with the predictor, whose list's count is counts[7])
+  const int batch = (n <= batch_cells<M::N1>() && !prof && !a.use_pred) ? BATCH_TRIPS : 1;
+  while (batch > 1 && trip < max_trips) {
+    const int k = (int)(max_trips - trip < batch ? max_trips - trip : batch);
+    for (int t = 0; t < k; ++t) {
+      PELE_TRY(enqueue_fixed_trip<M>(a, cur, stream, true, 1));
+      cur = 1 - cur;
+    }
     PELE_TRY(hipMemcpyAsync(h_counts, a.counts, sizeof(h_counts), hipMemcpyDeviceToHost, stream));
     PELE_TRY(hipStreamSynchronize(stream));
+    trip += k;
+    if (h_counts[a.compact ? cur : 5] == 0) {
+      if (trips_out) *trips_out = (long)h_counts[7];
+      return hipSuccess;
+    }
+  }
+  // In the plain schedule the evaluation covers every cell whatever the counts say, so it is
+  // issued before the host waits for them: the wait (35 us of idle GPU) runs beside it.
+  const bool ahead = !a.compact && !prof && plan.host_counts && plan.counted;
+  for (; trip < max_trips; ++trip) {
+    unsigned int* const hc = ahead ? plan.host_counts : h_counts;
+    PELE_TRY(hipMemcpyAsync(hc, a.counts, sizeof(h_counts), hipMemcpyDeviceToHost, stream));
+    if (ahead) {
+      PELE_TRY(hipEventRecord(plan.counted, stream));
+      hipLaunchKernelGGL(k_trip_start, dim3(1), dim3(64), 0, stream, a.counts, 5, 5, 2 + (1 - cur), 0);
+      PELE_TRY(hipGetLastError());
+      hipLaunchKernelGGL(k_eval<M>, dim3(nb), dim3(64), 0, stream, a, a.list[1], &a.counts[4]);
+      PELE_TRY(hipGetLastError());
+      PELE_TRY(hipEventSynchronize(plan.counted));
+      for (int i = 0; i < 8; ++i) h_counts[i] = hc[i];
+    } else {
+      PELE_TRY(hipStreamSynchronize(stream));
+    }
     if (a.compact) {
       const unsigned int active = h_counts[cur];
       const unsigned int nsetup = h_counts[2 + cur];
       if (active == 0) break;
       const int nxt = 1 - cur;
-      hipLaunchKernelGGL(k_zero_two, dim3(1), dim3(64), 0, stream, a.counts, nxt, 2 + nxt);
-      PELE_TRY(hipGetLastError());
-      hipLaunchKernelGGL(k_zero_two, dim3(1), dim3(64), 0, stream, a.counts, 6, 6);
+      hipLaunchKernelGGL(k_trip_start, dim3(1), dim3(64), 0, stream, a.counts, cur, nxt, 2 + nxt, 0);
       PELE_TRY(hipGetLastError());
       const unsigned ga = (active + 63) / 64;
       if (a.use_pred && h_counts[7] > 0) {
@@ -3842,14 +3895,14 @@ hipError_t run_react_t(ReactArgs a, hipStream_t stream, long max_trips, long* tr
       if (h_counts[5] == 0) break;
       const unsigned int nsetup = h_counts[2 + cur];
       const int nxt = 1 - cur;
-      hipLaunchKernelGGL(k_zero_two, dim3(1), dim3(64), 0, stream, a.counts, 5, 2 + nxt);
-      PELE_TRY(hipGetLastError());
-      hipLaunchKernelGGL(k_zero_two, dim3(1), dim3(64), 0, stream, a.counts, 6, 6);
-      PELE_TRY(hipGetLastError());
-      PELE_TRY(tm.begin());
-      hipLaunchKernelGGL(k_eval<M>, dim3(nb), dim3(64), 0, stream, a, a.list[1], &a.counts[4]);
-      PELE_TRY(hipGetLastError());
-      PELE_TRY(tm.end(KK_EVAL, h_counts[5]));
+      if (!ahead) {
+        hipLaunchKernelGGL(k_trip_start, dim3(1), dim3(64), 0, stream, a.counts, 5, 5, 2 + nxt, 0);
+        PELE_TRY(hipGetLastError());
+        PELE_TRY(tm.begin());
+        hipLaunchKernelGGL(k_eval<M>, dim3(nb), dim3(64), 0, stream, a, a.list[1], &a.counts[4]);
+        PELE_TRY(hipGetLastError());
+        PELE_TRY(tm.end(KK_EVAL, h_counts[5]));
+      }
       if (nsetup > 0) {
         PELE_TRY(tm.begin());
         hipLaunchKernelGGL(k_setup<M>, dim3((nsetup + 63) / 64), dim3(64), 0, stream, a, a.slist[cur],

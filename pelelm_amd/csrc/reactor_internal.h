@@ -120,6 +120,10 @@ struct MlpDev;
 struct TripPlan {
   int graph_trips = 0;
   hipStream_t capture_stream = nullptr;
+  // 8 words of pinned host memory and an event, both the reactor's: with them the host
+  // waits for a trip's counts while the trip's evaluation runs (null: it waits first)
+  unsigned int* host_counts = nullptr;
+  hipEvent_t counted = nullptr;
 };
 // pred: the learned predictor's device view, required when a.use_pred = 1
 hipError_t run_react(int mech, const ReactArgs& a, hipStream_t stream, long max_trips, long* trips_out,

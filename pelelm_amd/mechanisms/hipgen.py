@@ -155,44 +155,66 @@ def _element_shift(mech: M.Mechanism) -> list:
              sum(v * s.composition.get(e, 0) for e, v in zip(els, alpha))) for s in mech.species]
 
 
+# Up to this many species the coefficients are literals in the code, chosen by selects: a
+# launch on a few cells waits for each line of a table in turn (LiDryer's rates of 1,000
+# cells 9.4 us with tables, 8.1 with literals), and nine species' selects cost little.
+LITERAL_SPECIES = 16
+
+
 def gen_tables(mech: M.Mechanism) -> str:
-    """The constant-memory tables, [range][species][8]: NASA coefficients over the
+    """The constant-memory tables (none up to LITERAL_SPECIES species), [range][species][8]: NASA coefficients over the
     molecular weight (mixture sums), as they are (per species), and g/RT's (a0, a1/2,
     a2/6, a3/12, a4/20, a5, a6, shifted)."""
     cn = _cname(mech.name)
-    shift = _element_shift(mech)
+    if mech.nspec <= LITERAL_SPECIES:
+        return ""
     out = []
-
-    def table(name, row):
+    for name in ("mass", "nasa", "gibbs"):
         out.append(f"static __constant__ double {cn}_{name}[2][{mech.nspec}][8] = {{")
-        for side in (0, 1):
+        for side in _table_rows(mech, name):
             out.append(" {")
-            for k, s in enumerate(mech.species):
-                out.append("  {" + ", ".join(_d(v) for v in row(k, s, s.low if side == 0 else s.high)) + "},")
+            out += ["  {" + ", ".join(_d(v) for v in row) + "}," for row in side]
             out.append(" },")
         out.append("};")
-
-    table("mass", lambda k, s, a: [a[i] / mech.W[k] for i in range(6)] + [0.0, 0.0])
-    table("nasa", lambda k, s, a: [a[i] for i in range(7)] + [0.0])
-    table("gibbs", lambda k, s, a: [a[0], a[1] / 2.0, a[2] / 6.0, a[3] / 12.0, a[4] / 20.0, a[5] + shift[k][0],
-                                    a[6] + shift[k][1], 0.0])
     return "\n".join(out)
+
+
+def _table_rows(mech: M.Mechanism, name: str) -> list:
+    """[range][species] -> 8 values."""
+    shift = _element_shift(mech) if name == "gibbs" else None
+
+    def row(k, s, a):
+        if name == "mass":
+            return [a[i] / mech.W[k] for i in range(6)] + [0.0, 0.0]
+        if name == "nasa":
+            return [a[i] for i in range(7)] + [0.0]
+        return [a[0], a[1] / 2.0, a[2] / 6.0, a[3] / 12.0, a[4] / 20.0, a[5] + shift[k][0], a[6] + shift[k][1], 0.0]
+
+    return [[row(k, s, s.low if side == 0 else s.high) for k, s in enumerate(mech.species)] for side in (0, 1)]
 
 
 def gen_thermo_tables(mech: M.Mechanism) -> str:
     cn = _cname(mech.name)
     groups = list(_thermo_groups(mech).items())
+    literal = mech.nspec <= LITERAL_SPECIES
     out = []
 
-    def sided(body):
-        # body(k) for every species, u naming its table's range
+    def sided(table, body):
+        # body(k, t) for every species; t(i) is coefficient i of its row
+        if literal:
+            rows = _table_rows(mech, table)
+            out.append("  const bool up[] = {" + ", ".join(f"((range >> {g}) & 1u) != 0u" for g in range(len(groups))) + "};")
+            for g, (tmid, ks) in enumerate(groups):
+                for k in ks:
+                    out.append("  " + body(k, lambda i: f"(up[{g}] ? {_d(rows[1][k][i])} : {_d(rows[0][k][i])})", ""))
+            return
         for g, (tmid, ks) in enumerate(groups):
             out.append("#pragma unroll 1")
             out.append(f"  for (int r = 0; r < 2; ++r) if ((int)((range >> {g}) & 1u) == r) {{")
             # inside the branch the compiler knows r to be the lane's own bit: keep it scalar
             out.append("    const int u = PELE_UNIFORM(r);")
             for k in ks:
-                out.append("    " + body(k))
+                out.append("    " + body(k, lambda i: f"t[{i}]", f"const double* t = {cn}_{table}[u][{k}]; "))
             out.append("  }")
 
     out.append("// one bit per break temperature: T in its upper range")
@@ -203,27 +225,27 @@ def gen_thermo_tables(mech: M.Mechanism) -> str:
     out.append("static __device__ __forceinline__ void mix(const unsigned range, const double* __restrict__ w, "
                "double* __restrict__ A) {")
     out.append("  for (int j = 0; j < 6; ++j) A[j] = 0.0;")
-    sided(lambda k: f"{{ const double* t = {cn}_mass[u][{k}]; for (int j = 0; j < 6; ++j) A[j] += w[{k}] * t[j]; }}")
+    sided("mass", lambda k, t, row: "{ " + row + " ".join(f"A[{j}] += w[{k}] * {t(j)};" for j in range(6)) + " }")
     out.append("}")
     out.append("static __device__ __forceinline__ void thermo_cph(const double T, double* __restrict__ cpR, "
                "double* __restrict__ hRT) {")
     out.append("  const double iT = 1.0 / T;")
     out.append("  const unsigned range = mech_" + cn + "::range(T);")
-    sided(lambda k: f"{{ const double* t = {cn}_nasa[u][{k}];"
-                    f" cpR[{k}] = t[0] + T * (t[1] + T * (t[2] + T * (t[3] + T * t[4])));"
-                    f" hRT[{k}] = t[0] + T * (0.5 * t[1] + T * ((1.0 / 3.0) * t[2] + T * (0.25 * t[3] + T * (0.2 * t[4]))))"
-                    f" + t[5] * iT; }}")
+    sided("nasa", lambda k, t, row: f"{{ {row}"
+          f"const double a0 = {t(0)}, a1 = {t(1)}, a2 = {t(2)}, a3 = {t(3)}, a4 = {t(4)};"
+          f" cpR[{k}] = a0 + T * (a1 + T * (a2 + T * (a3 + T * a4)));"
+          f" hRT[{k}] = a0 + T * (0.5 * a1 + T * ((1.0 / 3.0) * a2 + T * (0.25 * a3 + T * (0.2 * a4)))) + {t(5)} * iT; }}")
     out.append("}")
     out.append("static __device__ __forceinline__ void thermo_dcp(const double T, double* __restrict__ dcpR) {")
     out.append("  const unsigned range = mech_" + cn + "::range(T);")
-    sided(lambda k: f"{{ const double* t = {cn}_nasa[u][{k}];"
-                    f" dcpR[{k}] = t[1] + T * (2.0 * t[2] + T * (3.0 * t[3] + T * (4.0 * t[4]))); }}")
+    sided("nasa", lambda k, t, row: f"{{ {row}"
+          f"dcpR[{k}] = {t(1)} + T * (2.0 * {t(2)} + T * (3.0 * {t(3)} + T * (4.0 * {t(4)}))); }}")
     out.append("}")
     out.append("static __device__ __forceinline__ void gibbs(const double T, const double logT, double* __restrict__ gRT) {")
     out.append("  const double iT = 1.0 / T, l1 = 1.0 - logT;")
     out.append("  const unsigned range = mech_" + cn + "::range(T);")
-    sided(lambda k: f"{{ const double* t = {cn}_gibbs[u][{k}];"
-                    f" gRT[{k}] = t[0] * l1 - T * (t[1] + T * (t[2] + T * (t[3] + T * t[4]))) + t[5] * iT - t[6]; }}")
+    sided("gibbs", lambda k, t, row: f"{{ {row}"
+          f"gRT[{k}] = {t(0)} * l1 - T * ({t(1)} + T * ({t(2)} + T * ({t(3)} + T * {t(4)}))) + {t(5)} * iT - {t(6)}; }}")
     out.append("}")
     return "\n".join(out)
 
