@@ -157,7 +157,7 @@ def _element_shift(mech: M.Mechanism) -> list:
 
 # Up to this many species the coefficients are literals in the code, chosen by selects: a
 # launch on a few cells waits for each line of a table in turn (LiDryer's rates of 1,000
-# cells 9.4 us with tables, 8.1 with literals), and nine species' selects cost little.
+# cells 9.4 us with tables, 7.6 with literals), and nine species' selects cost little.
 LITERAL_SPECIES = 16
 
 
