@@ -7,11 +7,13 @@
  * the absolute tolerances, asked to react boxes, closed at teardown.  Every entry point
  * takes plain pointers and sizes; device arrays are HIP device pointers and all work is
  * enqueued on the caller's HIP stream.  The host-driven schedules (plain, queue, auto)
- * read the work-list counts back once per trip, so react returns with the integration
- * finished (the reference's caller synchronises right after the call anyway,
- * Source/PeleLM.cpp:5773-5775); the persistent schedule enqueues one kernel and
- * synchronises only to read the failure count under mi.on_fail = abort (never under
- * stream capture).
+ * read the work-list counts back once per trip (small boxes once per eight trips, captured
+ * graphs once per graph), and react returns with every kernel of the integration finished
+ * (the reference's caller synchronises right after the call anyway,
+ * Source/PeleLM.cpp:5773-5775), so the next call may use another stream; the persistent
+ * schedule and ReactorRK64 enqueue one kernel and synchronise only to read the failure
+ * count under mi.on_fail = abort (never under stream capture): a next call on another
+ * stream must be ordered behind them by the caller, since both use the reactor's workspace.
  *
  * Units are CGS in and out, as the reference converts before and after the call
  * (Source/PeleLM.cpp:5737-5746, 5764-5771).

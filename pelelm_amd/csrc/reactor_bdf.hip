@@ -3768,6 +3768,7 @@ hipError_t run_trips_graph(const ReactArgs& a, hipStream_t stream, long max_trip
     else
       hipLaunchKernelGGL(k_abandon<M>, dim3(nb), dim3(64), 0, stream, a, a.list[1], &a.counts[4]);
     PELE_TRY(hipGetLastError());
+    PELE_TRY(hipStreamSynchronize(stream));   // as in run_react_t: nothing outlives the call
   }
   if (trips_out) *trips_out = trip;
   return hipSuccess;
@@ -3931,6 +3932,11 @@ hipError_t run_react_t(ReactArgs a, hipStream_t stream, long max_trips, long* tr
       hipLaunchKernelGGL(k_abandon<M>, dim3(nb), dim3(64), 0, stream, a, a.list[1], &a.counts[4]);
     PELE_TRY(hipGetLastError());
   }
+  // Nothing outlives the call.  The evaluation issued ahead of the counts that ended the
+  // loop, and the last kernels under the cap on trips, read the workspace and append to the
+  // lists; the next call may use both on another stream, which nothing orders behind this
+  // one (a cell it has started by then would be appended twice, beyond the list's end).
+  if (ahead || trip == max_trips) PELE_TRY(hipStreamSynchronize(stream));
   if (trips_out) *trips_out = trip;
   PELE_TRY(tm.collect());
   return hipSuccess;
