@@ -263,6 +263,193 @@ __device__ __forceinline__ double hy2t(const double h, const double* w, double T
   return T;
 }
 
+// ---------------------------------------------------------------------------
+// The rates and the Jacobian reaction by reaction, from the mechanism's tables.  The
+// generated forms multiply exp(+-g/RT) of single species, where only the difference over a
+// reaction is bounded; below M::T_LOW (105 to 210 K, by mechanism) and above
+// M::T_HIGH such products can leave a double's range, to infinity or silently to zero.
+// There each reaction takes exponentials of its own: of its rate constant, and of that one's
+// exponent plus the difference of g/RT for the way back, which stays moderate where either
+// alone does not.  Loops over reactions stay rolled, with the arrays they index in scratch
+// memory: what counts is that the usual path keeps its registers (the callers pass copies),
+// not the speed of this one.
+// ---------------------------------------------------------------------------
+template <class M>
+struct Reaction {
+  const int* x;                     // its table row
+  double fwd, rev;                  // rate constants without third bodies (rev 0: one way)
+  double phi, dphidT, dphidM;       // third-body or fall-off factor, its derivatives
+  double pf, pr;                    // products of concentrations over either side
+  double dlnkf, dlnKc;              // d/dT of ln fwd and ln K_c
+  // h: enthalpies over RT, or null (dlnKc is then not formed)
+  __device__ __forceinline__ Reaction(const int j, const double* C, const double Ctot, const double T,
+                                      const double logT, const double invT, const double* g, const double* h)
+      : x(M::rx_int(j)), pf(1.0), pr(1.0) {
+    double dG = 0.0, dH = 0.0;
+    int dnu = 0;
+#pragma unroll 1
+    for (int s = 0; s < M::RX_SIDE; ++s) {
+      const int a = x[4 + s], b = x[4 + M::RX_SIDE + s];
+      if (a >= 0) {
+        pf *= C[a];
+        dG -= g[a];
+        if (h) dH -= h[a];
+        --dnu;
+      }
+      if (b >= 0) {
+        pr *= C[b];
+        dG += g[b];
+        if (h) dH += h[b];
+        ++dnu;
+      }
+    }
+    const double* d = M::rx_num(j);
+    const double e = d[1] + d[2] * logT - d[3] * invT;
+    fwd = d[0] * exp(e);
+    dlnkf = (d[2] + d[3] * invT) * invT;
+    rev = 0.0;
+    dlnKc = (dH - dnu) * invT;
+    if (x[1]) {
+      const double refC = (M::PATM / M::RU) * invT, ref = dnu > 0 ? 1.0 / refC : refC;
+      rev = d[0] * exp(e + dG);
+#pragma unroll 1
+      for (int s = dnu < 0 ? -dnu : dnu; s > 0; --s) rev *= ref;
+    }
+    phi = 1.0;
+    dphidT = dphidM = 0.0;
+    if (x[0] == 0) return;
+    double Mc = Ctot;
+#pragma unroll 1
+    for (int n = x[2]; n < x[3]; ++n) Mc += M::eff_e(n) * C[M::eff_k(n)];
+    if (x[0] == 1) {
+      phi = Mc;
+      dphidM = 1.0;
+      return;
+    }
+    const double dPrdM = d[4] / d[0] * exp(d[5] + d[6] * logT - d[7] * invT - e), Pr = dPrdM * Mc;
+    const double dPrdT = Pr * ((d[6] + d[7] * invT) * invT - dlnkf);
+    double F = 1.0, dFdPr = 0.0, dFdT = 0.0;
+    if (x[0] == 3) {
+      const double e3 = d[8] * exp(d[9] * T), e1 = d[10] * exp(d[11] * T), e2 = d[12] * exp(-d[13] * invT);
+      double Fc = e3 + e1 + e2, dFc = d[9] * e3 + d[11] * e1 + d[13] * invT * invT * e2;
+      if (Fc < 1e-300) {
+        Fc = 1e-300;
+        dFc = 0.0;
+      }
+      const double logFc = log10(Fc), cc = -0.4 - 0.67 * logFc, nn = 0.75 - 1.27 * logFc;
+      const double PrS = fmax(Pr, 1e-300);
+      const double u = log10(PrS) + cc, dd = nn - 0.14 * u, f1 = u / dd, den = 1.0 + f1 * f1;
+      F = exp(2.302585092994045684 * logFc / den);
+      const double df1du = nn / (dd * dd), df1dl = (-0.67 * dd + 1.1762 * u) / (dd * dd);
+      const double slope = -logFc * 2.0 * f1 / (den * den);
+      dFdPr = F * slope * df1du / PrS;
+      dFdT = F * (1.0 / den + slope * df1dl) * dFc / Fc;
+    }
+    const double gg = Pr / (1.0 + Pr), dg = 1.0 / ((1.0 + Pr) * (1.0 + Pr));
+    phi = gg * F;
+    dphidM = (dg * F + gg * dFdPr) * dPrdM;
+    dphidT = (dg * F + gg * dFdPr) * dPrdT + gg * dFdT;
+  }
+  __device__ __forceinline__ double net() const { return fwd * pf - rev * pr; }
+  // the species the reaction makes or takes (-1 beyond the last) and how many of it
+  __device__ __forceinline__ int species(const int s) const { return x[4 + 2 * M::RX_SIDE + s]; }
+  __device__ __forceinline__ double change(const int s) const { return x[4 + 4 * M::RX_SIDE + s]; }
+};
+
+template <class M>
+__device__ __forceinline__ void wdot_by_reaction(const double* C, const double T, const double logT, const double invT,
+                                                 const double* g, double* wd) {
+  double Ctot = 0.0;
+#pragma unroll 1
+  for (int k = 0; k < M::NS; ++k) {
+    wd[k] = 0.0;
+    Ctot += C[k];
+  }
+#pragma unroll 1
+  for (int j = 0; j < M::NR; ++j) {
+    const Reaction<M> r(j, C, Ctot, T, logT, invT, g, nullptr);
+    const double q = r.phi * r.net();
+#pragma unroll 1
+    for (int s = 0; s < 2 * M::RX_SIDE && r.species(s) >= 0; ++s) wd[r.species(s)] += r.change(s) * q;
+  }
+}
+// net molar production rates at any temperature.  Each branch forms g/RT for itself: across
+// the branch it would hold two registers per species beside the concentrations'.
+template <class M>
+__device__ __forceinline__ void net_rates(const double* __restrict__ C, const double T, double* __restrict__ wd) {
+  constexpr int N = M::NS;
+  const double logT = log(T), invT = 1.0 / T;
+  if (T < M::T_LOW || T > M::T_HIGH) {
+    double c[N], g[N], w[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) c[k] = C[k];
+    M::gibbs(T, logT, g);
+    wdot_by_reaction<M>(c, T, logT, invT, g, w);
+#pragma unroll
+    for (int k = 0; k < N; ++k) wd[k] = w[k];
+  } else {
+    double g[N];
+    M::gibbs(T, logT, g);
+    M::wdot(C, T, logT, invT, g, wd);
+  }
+}
+
+// wd, dwd/dT and, in at(i, k) for i, k < NS, the derivatives d(W_i wd_i)/d(rhoY_k)
+template <class M, class At>
+__device__ __forceinline__ void jacobian_by_reaction(const double* C, const double T, const double logT,
+                                                     const double invT, const double* g, const double* h, double* wd,
+                                                     double* dwdT, const At& at) {
+  constexpr int N = M::NS;
+  double Ctot = 0.0;
+#pragma unroll 1
+  for (int k = 0; k < N; ++k) {
+    wd[k] = dwdT[k] = 0.0;
+    Ctot += C[k];
+#pragma unroll 1
+    for (int i = 0; i < N; ++i) at(i, k) = 0.0;
+  }
+#pragma unroll 1
+  for (int j = 0; j < M::NR; ++j) {
+    const Reaction<M> r(j, C, Ctot, T, logT, invT, g, h);
+    const int* x = r.x;
+    const double net = r.net(), q = r.phi * net;
+    const double dqdT = r.dphidT * net + r.phi * (r.dlnkf * net + r.rev * r.pr * r.dlnKc);
+    // d = dq/dC_k goes to the rows of the species that the reaction makes or takes (not of
+    // one on both sides: what it gains and loses would leave a rounding error in its row)
+    auto column = [&](const int k, const double d) {
+      const double dk = d * M::imw(k);
+#pragma unroll 1
+      for (int s = 0; s < 2 * M::RX_SIDE && r.species(s) >= 0; ++s)
+        at(r.species(s), k) += r.change(s) * M::mw(r.species(s)) * dk;
+    };
+#pragma unroll 1
+    for (int s = 0; s < 2 * M::RX_SIDE && r.species(s) >= 0; ++s) {
+      wd[r.species(s)] += r.change(s) * q;
+      dwdT[r.species(s)] += r.change(s) * dqdT;
+    }
+#pragma unroll 1
+    for (int s = 0; s < M::RX_SIDE; ++s) {
+      const int a = x[4 + s], b = x[4 + M::RX_SIDE + s];
+      double pa = 1.0, pb = 1.0;   // the side without this factor
+#pragma unroll 1
+      for (int t = 0; t < M::RX_SIDE; ++t) {
+        const int u = x[4 + t], v = x[4 + M::RX_SIDE + t];
+        if (t != s && u >= 0) pa *= C[u];
+        if (t != s && v >= 0) pb *= C[v];
+      }
+      if (a >= 0) column(a, r.phi * r.fwd * pa);
+      if (b >= 0) column(b, -r.phi * r.rev * pb);
+    }
+    if (x[0]) {
+      const double tb = r.dphidM * net;
+#pragma unroll 1
+      for (int k = 0; k < N; ++k) column(k, tb);
+#pragma unroll 1
+      for (int e = x[2]; e < x[3]; ++e) column(M::eff_k(e), M::eff_e(e) * tb);
+    }
+  }
+}
+
 template <class M>
 __device__ __forceinline__ void rhs(const double* __restrict__ y, const double t, const WS& ws, const double rE0,
                                     const double fH, double* __restrict__ f, double& Tsol, int* hy2t_iters = nullptr) {
@@ -272,12 +459,10 @@ __device__ __forceinline__ void rhs(const double* __restrict__ y, const double t
   const double T = hy2t<M>(rE0 + fH * t, y, y[N], A, hy2t_iters);   // per volume: rho h of rhoY
   Tsol = T;
   const double rhocp = M::RU * mix_cp(A, T);
-  const double logT = log(T), invT = 1.0 / T;
-  double C[N], g[N], wd[N];
+  double C[N], wd[N];
 #pragma unroll
   for (int k = 0; k < N; ++k) C[k] = y[k] * M::imw(k);
-  M::gibbs(T, logT, g);
-  M::wdot(C, T, logT, invT, g, wd);
+  net_rates<M>(C, T, wd);
 #pragma unroll
   for (int k = 0; k < N; ++k) f[k] = wd[k] * M::mw(k) + ws[S::FY + k];
   // energy closure from rho h = sum_k rhoY_k h_k(T): rho cp dT/dt = F_h - sum_k h_k d(rhoY_k)/dt
@@ -292,10 +477,20 @@ __device__ __forceinline__ void rhs(const double* __restrict__ y, const double t
 // entries are produced.
 // The tiles come by value: by reference their addresses are reloaded from the stack after
 // every store of an entry, which may alias them.
-template <class M>
-__device__ __noinline__ void jacobian(const double* __restrict__ y, const double T, const double fT, const WS ws,
-                                      const WS js) {
+// TABLES: the form outside M::T_LOW .. M::T_HIGH, a function of its own.  Up to 32 unknowns
+// the usual one hands over to it, above the caller chooses: with two calls in the set-up
+// kernel LiDryer 16^3 took 4.50 ms instead of 4.04, while a hand-over cost the boxes of 53
+// to 88 species 0.6 to 1.4 % (the 56-species 33 x 31 x 29 box 101.6 ms against 100.1).
+template <class M, bool TABLES>
+__device__ __noinline__ void jacobian_in(const double* __restrict__ y, const double T, const double fT, const WS ws,
+                                         const WS js) {
   constexpr int N = M::NS, N1 = M::N1;
+  if constexpr (!TABLES && N1 <= 32) {
+    if (T < M::T_LOW || T > M::T_HIGH) {
+      jacobian_in<M, true>(y, T, fT, ws, js);
+      return;
+    }
+  }
   auto at = [&](int i, int k) -> double& { return js[Slots<N1>::JS + i * N1 + k]; };
   using S = Slots<N1>;
   const double logT = log(T), invT = 1.0 / T;
@@ -310,16 +505,27 @@ __device__ __noinline__ void jacobian(const double* __restrict__ y, const double
   rhocp *= M::RU;
   // T row: fT = (F_h - R T sum_i hRT_i (wdot_i + F_Y,i / W_i)) / rhocp (fT is passed in);
   // d fT / d rhoY_k = (-R T sum_i hRT_i/W_i J_ik - fT cp_k) / rhocp, the forcing being constant
-  double s = 0.0;
-  M::jacobian(C, T, logT, invT, g, hRT, wd, dwdT,
-              [&](int i, int k, double v) {
-                at(i, k) = v;
-                s += hRT[i] * M::imw(i) * v;
-              },
-              [&](int k) {
-                at(N, k) = (-M::RU * T * s - fT * M::RU * cpR[k] * M::imw(k)) / rhocp;
-                s = 0.0;
-              });
+  if constexpr (TABLES) {
+    jacobian_by_reaction<M>(C, T, logT, invT, g, hRT, wd, dwdT, at);
+#pragma unroll 1
+    for (int k = 0; k < N; ++k) {
+      double s = 0.0;
+#pragma unroll 1
+      for (int i = 0; i < N; ++i) s += hRT[i] * M::imw(i) * at(i, k);
+      at(N, k) = (-M::RU * T * s - fT * M::RU * cpR[k] * M::imw(k)) / rhocp;
+    }
+  } else {
+    double s = 0.0;
+    M::jacobian(C, T, logT, invT, g, hRT, wd, dwdT,
+                [&](int i, int k, double v) {
+                  at(i, k) = v;
+                  s += hRT[i] * M::imw(i) * v;
+                },
+                [&](int k) {
+                  at(N, k) = (-M::RU * T * s - fT * M::RU * cpR[k] * M::imw(k)) / rhocp;
+                  s = 0.0;
+                });
+  }
   double dcp[N];
   M::thermo_dcp(T, dcp);
   double drhocp = 0.0, sTT = 0.0;
@@ -331,6 +537,12 @@ __device__ __noinline__ void jacobian(const double* __restrict__ y, const double
   }
   drhocp *= M::RU;
   at(N, N) = (-M::RU * sTT - fT * drhocp) / rhocp;
+}
+template <class M>
+__device__ __forceinline__ void jacobian(const double* __restrict__ y, const double T, const double fT, const WS& ws,
+                                         const WS& js) {
+  if (M::N1 > 32 && (T < M::T_LOW || T > M::T_HIGH)) jacobian_in<M, true>(y, T, fT, ws, js);
+  else jacobian_in<M, false>(y, T, fT, ws, js);
 }
 template <class M>
 __device__ __forceinline__ void jacobian(const double* __restrict__ y, const double T, const double fT, const WS& ws) {
@@ -2996,6 +3208,23 @@ __global__ void k_plain_counts(unsigned int* counts, unsigned int n) {
   }
 }
 
+// a cell's rates outside M::T_LOW .. M::T_HIGH, from and to its arrays: a function that the
+// rates kernel leaves by (its table loops inlined, or a way back into the kernel, cost the
+// rates of drm19 128^3 0.515 ms against 0.502)
+template <class M>
+__device__ __noinline__ void rates_by_reaction(const double* rhoY, const long ys, const double rscale, const double T,
+                                               double* rdot, const long ds, const double oscale) {
+  constexpr int N = M::NS;
+  const double logT = log(T);
+  double C[N], g[N], wd[N];
+#pragma unroll 1
+  for (int n = 0; n < N; ++n) C[n] = rscale * rhoY[n * ys] * M::imw(n);
+  M::gibbs(T, logT, g);
+  wdot_by_reaction<M>(C, T, logT, 1.0 / T, g, wd);
+#pragma unroll 1
+  for (int n = 0; n < N; ++n) rdot[n * ds] = wd[n] * M::mw(n) * oscale;
+}
+
 // net production rates rho*wdot (g/cm^3/s) with T re-solved from h
 // reactionRateRhoY per cell (Source/PeleLM_K.H:57-98): rho = sum_k rhoY_k, Y = rhoY / rho,
 // h = rhoH / rho x hscale (solved per volume, so that rho drops out), T = HY2T(h, Y)
@@ -3028,6 +3257,10 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(PELE_RATES_WAVES(M::N1))
   // per volume: rho h = sum_k rhoY_k h_k(T)
   const double Tc = hy2t<M>(rhoH.p[cell_off(rhoH, i, j, k)] * hscale, Y, T.p[cell_off(T, i, j, k)], A);
   if (Tout) Tout[c] = Tc;
+  if (Tc < M::T_LOW || Tc > M::T_HIGH) {
+    rates_by_reaction<M>(rhoY.p + oy, rhoY.ns, rscale, Tc, rdot.p + cell_off(rdot, i, j, k), rdot.ns, oscale);
+    return;
+  }
   const double logT = log(Tc), invT = 1.0 / Tc;
   double C[N], g[N], wd[N];
 #pragma unroll
@@ -3067,12 +3300,10 @@ __global__ void __launch_bounds__(64) PELE_WAVES_PER_EU(PELE_EVAL_WAVES(M::N1)) 
 #pragma unroll
     for (int n = 0; n < N; ++n) y[n] = a.rY.p[oy + n * a.rY.ns];
     const double T = hy2t<M>(a.rE.p[cell_off(a.rE, i, j, k)], y, a.T.p[cell_off(a.T, i, j, k)], A);
-    const double logT = log(T), invT = 1.0 / T;
-    double C[N], g[N], wd[N];
+    double C[N], wd[N];
 #pragma unroll
     for (int n = 0; n < N; ++n) C[n] = y[n] * M::imw(n);
-    M::gibbs(T, logT, g);
-    M::wdot(C, T, logT, invT, g, wd);
+    net_rates<M>(C, T, wd);
     double kmax = 0.0;
     const long of = a.rYsrc.p ? cell_off(a.rYsrc, i, j, k) : 0;
 #pragma unroll

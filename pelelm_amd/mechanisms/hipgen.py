@@ -130,8 +130,8 @@ def _element_shift(mech: M.Mechanism) -> list:
     """(d5, d6) per species: what to add to the NASA coefficients a5 and a6 so that g/RT
     loses sum_e n_ke (alpha_e + beta_e / T).  A reaction that conserves its elements does
     not see it, while exp(g/RT) of every species, and the product over either side of a
-    reaction, stays within the range of a double down to 200 K, as the exponential of the
-    reaction's own difference does.  alpha and beta are the least-squares fit of g/RT over
+    reaction, stays within the range of a double down to the cold end that ``shared_range``
+    finds (105 to 210 K).  alpha and beta are the least-squares fit of g/RT over
     200 - 4000 K, rounded (1, and 10 K)."""
     els = list(mech.elements)
     for r in mech.reactions:
@@ -177,6 +177,116 @@ def gen_tables(mech: M.Mechanism) -> str:
             out.append(" },")
         out.append("};")
     return "\n".join(out)
+
+
+# The shared form (gen_wdot_shared) multiplies exponentials that a reaction's own difference
+# would have cancelled, so it stands only where every product of them, partial ones
+# included, is within exp(+-SHARED_LIMIT): what is left of a double's exp(+-709) is for the
+# concentrations, whose products may then be as small as 1e-60 (1e-138 at 298 K in the
+# mechanism that needs most).  A lower limit moves the line up into temperatures that
+# forced cells reach: at 480 (250 K for the 56-species mechanism) a box of 33 x 31 x 29 such
+# cells took 29 ms in k_eval against 11, the few cold lanes making their waves take both
+# forms.
+SHARED_LIMIT = 570.0
+
+
+def shared_range(mech: M.Mechanism) -> tuple:
+    """(low, high): the temperatures between which the shared form's exponentials and
+    their products stay within SHARED_LIMIT, on a grid of 5 K below 3500 K and 100 K above,
+    at most 20000 K.  Outside, the rates take one exponential per reaction."""
+    shift = _element_shift(mech)
+
+    def holds(T):
+        logT = math.log(T)
+        g = []
+        for s, (d5, d6) in zip(mech.species, shift):
+            a = s.low if T < s.T[1] else s.high
+            g.append(a[0] * (1.0 - logT) - a[1] * T / 2 - a[2] * T ** 2 / 6 - a[3] * T ** 3 / 12 - a[4] * T ** 4 / 20
+                     + (a[5] + d5) / T - (a[6] + d6))
+        for r in mech.reactions:
+            if abs(r.beta * logT - r.Ea / M.R_CAL / T) > SHARED_LIMIT:
+                return False
+            for side in (r.reactants, r.products):
+                t = 0.0
+                for i, c in sorted(side.items()):
+                    for _ in range(c):
+                        t += g[i]
+                        if abs(t) > SHARED_LIMIT:
+                            return False
+        return all(abs(x) <= SHARED_LIMIT for x in g)
+
+    low, high = 3500.0, 3500.0
+    while low > 5.0 and holds(low - 5.0):
+        low -= 5.0
+    while high < 20000.0 and holds(high + 100.0):
+        high += 100.0
+    return low, high
+
+
+def gen_reaction_tables(mech: M.Mechanism) -> str:
+    """The reactions as tables, for the rates and Jacobian outside the shared form's range.
+    Integers: kind (0 elementary, 1 three-body, 2 Lindemann, 3 Troe), reversible, first and
+    last + 1 of the efficiencies, then the species of either side, each as often as its
+    coefficient, -1 beyond; the species whose coefficients differ between the sides, -1
+    beyond, and by how much.  Numbers: f, x, b, Ta of the rate constant f exp(x + b ln T -
+    Ta / T) and of the low-pressure one, then Fcent = c3 exp(-T/T3) + c1 exp(-T/T1) + c2
+    exp(-T2/T) as (c3, -1/T3, c1, -1/T1, c2, T2).  Efficiencies: species, and e - 1."""
+    cn = _cname(mech.name)
+    width = max(sum(s.values()) for r in mech.reactions for s in (r.reactants, r.products))
+    ints, nums, eff_k, eff_e = [], [], [], []
+
+    def arrhenius(A, b, Ea):   # a constant is kept as it is, as _kf_expr writes it
+        return [A, 0.0, 0.0, 0.0] if b == 0.0 and Ea == 0.0 else [1.0, math.log(A), b, Ea / M.R_CAL]
+
+    for r in mech.reactions:
+        first = len(eff_k)
+        if r.has_third_body:
+            for k, e in sorted(r.efficiencies.items()):
+                if e != 1.0:
+                    eff_k.append(k)
+                    eff_e.append(e - 1.0)
+        kind = {"elementary": 0, "three-body": 1, "falloff": 2 if r.troe is None else 3}[r.kind]
+        row = [kind, int(r.reversible), first, len(eff_k)]
+        for side in (r.reactants, r.products):
+            ks = [i for i, c in sorted(side.items()) for _ in range(c)]
+            row += ks + [-1] * (width - len(ks))
+        net = {k: r.products.get(k, 0) - r.reactants.get(k, 0) for k in sorted({**r.reactants, **r.products})}
+        net = [(k, v) for k, v in net.items() if v != 0]
+        for j in (0, 1):
+            row += [kv[j] for kv in net] + [-1] * (2 * width - len(net))
+        ints.append(row)
+        f = [0.0] * 6
+        if r.troe is not None:
+            a, T3, T1 = r.troe[:3]
+            if T3 > 1e-20:
+                f[0], f[1] = 1.0 - a, -1.0 / T3
+            f[2], f[3] = a, (0.0 if T1 >= 1e20 else -1.0 / T1)
+            if len(r.troe) == 4:
+                f[4], f[5] = 1.0, r.troe[3]
+        nums.append(arrhenius(r.A, r.beta, r.Ea) + arrhenius(*(r.low or (1.0, 0.0, 0.0))) + f)
+    out = [f"static __constant__ int {cn}_rx_int[{mech.nreac}][{4 + 6 * width}] = {{"]
+    out += ["  {" + ", ".join(str(v) for v in row) + "}," for row in ints]
+    out.append("};")
+    out.append(f"static __constant__ double {cn}_rx_num[{mech.nreac}][14] = {{")
+    out += ["  {" + ", ".join(_d(v) for v in row) + "}," for row in nums]
+    out.append("};")
+    out.append(f"static __constant__ int {cn}_eff_k[] = {{" + ", ".join(str(k) for k in eff_k or [0]) + "};")
+    out.append(f"static __constant__ double {cn}_eff_e[] = {{" + ", ".join(_d(e) for e in eff_e or [0.0]) + "};")
+    return "\n".join(out)
+
+
+def gen_reaction_access(mech: M.Mechanism) -> str:
+    cn = _cname(mech.name)
+    width = max(sum(s.values()) for r in mech.reactions for s in (r.reactants, r.products))
+    low, high = shared_range(mech)
+    return "\n".join([
+        "// temperatures between which wdot and jacobian hold; outside, the reaction tables",
+        f"static constexpr double T_LOW = {_d(low)}, T_HIGH = {_d(high)};",
+        f"static constexpr int RX_SIDE = {width};",
+        f"static __device__ __forceinline__ const int* rx_int(int j) {{ return {cn}_rx_int[j]; }}",
+        f"static __device__ __forceinline__ const double* rx_num(int j) {{ return {cn}_rx_num[j]; }}",
+        f"static __device__ __forceinline__ int eff_k(int e) {{ return {cn}_eff_k[e]; }}",
+        f"static __device__ __forceinline__ double eff_e(int e) {{ return {cn}_eff_e[e]; }}"])
 
 
 def _table_rows(mech: M.Mechanism, name: str) -> list:
@@ -662,7 +772,7 @@ def write_inc(mech: M.Mechanism, path: str) -> None:
     cn = _cname(name)
     lines = [f"// GENERATED by pelelm_amd/mechanisms/hipgen.py from {name}.yaml -- do not edit.",
              f"// {ns} species, {mech.nreac} reactions.", "#pragma once", "",
-             gen_tables(mech), "",
+             gen_tables(mech), "", gen_reaction_tables(mech), "",
              f"struct mech_{cn} {{", "",
              f"static constexpr int NS = {ns};", f"static constexpr int NR = {mech.nreac};",
              f"static constexpr int N1 = {ns + 1};",
@@ -697,6 +807,8 @@ def write_inc(mech: M.Mechanism, path: str) -> None:
     lines.append(gen_thermo_tables(mech))
     lines.append("")
     lines.append(gen_wdot_shared(mech))
+    lines.append("")
+    lines.append(gen_reaction_access(mech))
     lines.append("")
     lines.append(gen_jacobian(mech))
     lines.append("")
