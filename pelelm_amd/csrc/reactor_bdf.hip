@@ -746,6 +746,9 @@ struct Lane {
       for (int i = j + 2; i >= 2; --i) l[i] = l[i] * xi + l[i - 1];
     }
   }
+  // The change of order, and prepare_next_step below, as operations of their own on a history
+  // in the workspace: the component tests run these on the device, one by one.  A trip runs
+  // trip_end's pass, which tests/test_step_logic.py holds to the separate operations.
   __device__ void increase_bdf() {
     const double A1 = increase_coeffs();
 #pragma unroll
