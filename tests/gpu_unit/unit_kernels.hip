@@ -382,7 +382,8 @@ int unit_lu_t(int coop, int fp32, int sweeps, long n, const double* J, const dou
 #ifdef UNIT_HOST
   if (coop) return -2;   // lanes of the cooperative kernels cannot run one at a time
 #endif
-  // coop: 0 one lane per cell, 1 the cooperative LU, 2 the blocked LU on the matrix cores
+  // coop: 0 one lane per cell, 1 the cooperative LU, 2 the blocked LU on the matrix cores,
+  // 3 the cooperative LU that solves its first system itself (the solve kernel does not run)
   const long nw = (n + 63) / 64;
   double *dJ = dev_copy(J, n * N1 * N1), *dg = dev_copy(gamma, n), *db = dev_copy(b, n * N1);
   double* de = dev_copy(ewt, n * N1);
@@ -409,6 +410,7 @@ int unit_lu_t(int coop, int fp32, int sweeps, long n, const double* J, const dou
   a.ir_tol = 1e-4;
   a.lu_lane = coop ? 0 : 1;
   a.lu_mfma = coop == 2 ? 1 : 0;
+  a.fuse = coop == 3 ? 1 : 0;
   hipLaunchKernelGGL(k_lu_prep<M>, dim3((unsigned)nw), dim3(64), 0, nullptr, dJ, dg, dp, db, de, ws, mats, n);
   hcounts[0] = (unsigned)n;
   UNIT_H2D(dcount, hcounts, sizeof(hcounts));
@@ -426,7 +428,7 @@ int unit_lu_t(int coop, int fp32, int sweeps, long n, const double* J, const dou
   UNIT_D2H(hs.data(), ds, n * sizeof(double));
   std::vector<int> sl;
   for (long i = 0; i < n; ++i)
-    if (pend[i] && hs[i] == 0.0) sl.push_back((int)i);
+    if (pend[i] && hs[i] == 0.0 && coop != 3) sl.push_back((int)i);
   int* dsl = dev_copy(sl.empty() ? ident.data() : sl.data(), sl.empty() ? 1 : (long)sl.size());
   hcounts[6] = (unsigned)sl.size();
   UNIT_H2D(dcount, hcounts, sizeof(hcounts));

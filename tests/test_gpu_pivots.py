@@ -8,8 +8,10 @@ the search by upper words must settle on the lower ones.
 """
 import numpy as np
 import pytest
+import torch   # before the unit library: a process takes its HIP runtime from the first of the two
 
 import test_gpu_unit as U
+from pelelm_amd import cells, reactor
 
 
 def _matrix(rng, n1, kind):
@@ -62,3 +64,73 @@ def test_pivot_order_with_ties(mech, n1, kind):
             # condition number below 10: a few hundred rounding errors of the solution
             xe = np.linalg.solve(m[c], b[c])
             assert np.max(np.abs(x[c] - xe)) <= 1e-12 * np.max(np.abs(xe))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mech,n1", [("LiDryer", 10), ("drm19", 22), ("dodecane53", 54)])
+def test_factorisation_solves_its_first_system(mech, n1):
+    """The solution that the cooperative factorisation forms from its registers: that of the
+    solve kernel and of numpy, on the pending cells alone (every fifth is idle, every seventh
+    singular: those keep what they held, 0)."""
+    rng = np.random.default_rng(100 + n1)
+    n = 131   # half a wave left over where two cells share one
+    m = np.eye(n1)[None] + rng.uniform(-0.5, 0.5, (n, n1, n1)) / np.sqrt(n1)
+    m = np.stack([a[rng.permutation(n1)] for a in m])
+    singular = np.arange(n) % 7 == 3
+    m[singular, :, n1 // 2] = 0.0
+    pend = (np.arange(n) % 5 != 0).astype(np.int32)
+    b = rng.normal(size=(n, n1))
+    J = np.ascontiguousarray(np.eye(n1)[None] - m)
+    m = np.eye(n1)[None] - J
+    G = U._load("libunit_gpu.so")
+    x, sing, lu, perm, _ = U.run_lu(G, mech, 3, J, np.ones(n), pend, b)
+    x1, sing1, lu1, perm1, _ = U.run_lu(G, mech, 1, J, np.ones(n), pend, b)
+    ok = (pend == 1) & ~singular
+    np.testing.assert_array_equal(sing, sing1)
+    np.testing.assert_array_equal(perm, perm1)
+    np.testing.assert_array_equal(lu, lu1)
+    assert np.all(sing[ok] == 0) and np.all(sing[(pend == 1) & singular] == n1 // 2 + 1)
+    assert np.all(x[~ok] == 0.0)
+    # condition numbers below 100: 1e4 rounding errors of the solution at most
+    xe = np.linalg.solve(m[ok], b[ok][..., None])[..., 0]
+    size = np.abs(xe).max(axis=1, keepdims=True)
+    assert np.linalg.cond(m[ok]).max() < 100.0
+    assert np.max(np.abs(x[ok] - xe) / size) < 1e-12
+    assert np.max(np.abs(x[ok] - x1[ok]) / size) < 1e-12
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("solve", ["denseAJ_direct", "GMRES"])
+@pytest.mark.parametrize("schedule", ["plain", "queue"])
+@pytest.mark.parametrize("wl,mech,limit", [("lidryer_16", "LiDryer", 4096), ("drm19_64", "drm19", 4096),
+                                           ("dodecane53_64_mix", "dodecane53", 2048)])
+def test_batched_trips_change_nothing(wl, mech, limit, schedule, solve):
+    """A box of the largest size whose trips come in batches, and the same cells with one more
+    (a copy of the first), whose trips come one by one: the same states, counts and trips,
+    with all cells done and with a cap on trips that is no multiple of a batch."""
+    d = cells.generate_workload(wl, ncell=limit)
+    got = {}
+    for n in (limit, limit + 1):
+        for cap in (0, 19):
+            r = reactor.ReactorBase.create("ReactorCvode")
+            for k, v in (("mi.mechanism", mech), ("ode.rtol", 1e-6), ("ode.atol", 1e-10), ("mi.schedule", schedule),
+                         ("cvode.solve_type", solve), ("mi.max_trips", cap), ("mi.on_fail", "continue")):
+                r.set(k, v)
+            r.init(2, n)
+            idx = np.arange(n) % limit
+            s = [torch.tensor(np.ascontiguousarray(d[k][..., idx]), device="cuda") for k in ("rY", "T", "rE")]
+            FC = torch.zeros(n, dtype=torch.float64, device="cuda")
+            r.react(s[0], None, s[1], s[2], None, FC, None, d["dt"])
+            torch.cuda.synchronize()
+            st = r.stats()
+            r.close()
+            got[n, cap] = [t.cpu().numpy()[..., :limit] for t in s + [FC]]
+            got[n, cap, "trips"] = st["ntrips"]
+            assert st["nfail"] == np.count_nonzero(FC.cpu().numpy() < 0)
+            # (without a cap, five Krylov vectors leave one cell of the 53-species mix unsolved)
+            assert st["nfail"] > 0 or cap == 0
+    for cap in (0, 19):
+        for a, b in zip(got[limit, cap], got[limit + 1, cap]):
+            np.testing.assert_array_equal(a, b)
+        assert got[limit, cap, "trips"] == got[limit + 1, cap, "trips"]
+    assert got[limit, 19, "trips"] == 19

@@ -42,7 +42,7 @@ def lib():
 
 def _react(lib, d, n, compact, gmres, ahead, cap):
     p = lambda a: a.ctypes.data_as(C.c_void_p)  # noqa: E731
-    rY, T, rE = (np.ascontiguousarray(d[k][..., :n]) for k in ("rY", "T", "rE"))
+    rY, T, rE = (d[k][..., :n].copy() for k in ("rY", "T", "rE"))
     FC, cnt, out = np.zeros(n), np.zeros(16, dtype=np.uint64), (C.c_long * 4)()
     rc = lib.host_react(C.c_long(n), p(rY), p(T), p(rE), p(FC), C.c_double(d["dt"]), C.c_double(1e-6),
                         C.c_double(1e-10), compact, gmres, ahead, C.c_long(cap), p(cnt), out)
@@ -67,3 +67,21 @@ def test_no_kernel_outlives_the_call(lib, box, n, compact, gmres, ahead, cap):
         assert out["trips"] == 19
         assert cnt[8] == np.count_nonzero(FC < 0) > 0
         assert np.abs(FC).max() <= 19
+
+
+@pytest.mark.parametrize("compact,gmres", [(0, 0), (1, 0), (0, 1), (1, 1)])
+@pytest.mark.parametrize("cap", [60100, 19])
+def test_batches_and_early_evaluations_change_nothing(lib, box, compact, gmres, cap):
+    """The same cells with their trips in batches of eight, one by one, and one by one with
+    the evaluation issued before the wait: the same states, counts and number of trips."""
+    runs = [_react(lib, box, LIMIT, compact, gmres, 0, cap)] + \
+        [_react(lib, box, LIMIT + 1, compact, gmres, ahead, cap) for ahead in (0, 1)]
+    batched, single, early = runs
+    for other in (single, early):
+        for a, b in zip(batched[:3], other[:3]):
+            np.testing.assert_array_equal(a[..., :LIMIT], b[..., :LIMIT])
+        assert batched[4]["trips"] == other[4]["trips"]
+    trips = batched[4]["trips"]
+    assert batched[4]["looks"] == -(-trips // 8)
+    assert single[4]["looks"] == early[4]["looks"] == trips + (cap != 19)
+    np.testing.assert_array_equal(single[3], early[3])
