@@ -132,7 +132,8 @@ def _element_shift(mech: M.Mechanism) -> list:
     not see it, while exp(g/RT) of every species, and the product over either side of a
     reaction, stays within the range of a double down to the cold end that ``shared_range``
     finds (105 to 210 K).  alpha and beta are the least-squares fit of g/RT over
-    200 - 4000 K, rounded (1, and 10 K)."""
+    200 - 4000 K, rounded (1, and 10 K).  A reaction that does not conserve them (the loader
+    refuses such a mechanism) leaves g/RT as it is; ``shared_range`` goes by the shift in use."""
     els = list(mech.elements)
     for r in mech.reactions:
         for e in els:

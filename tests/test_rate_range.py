@@ -207,3 +207,23 @@ def test_gpu_jacobian_is_right_down_to_80_K(name):
     J = U.run_jac_lu(U._load("libunit_gpu.so"), name, y3, T3, fT3, np.full(len(T3), 1e-30), np.zeros_like(y3))[0]
     for lane in (1, 2):
         _check_jacobian(mech, m, Cc, T, y, fT, J[lane::3])
+
+
+def test_range_follows_the_shift_in_use():
+    """A reaction that does not conserve the elements leaves the mechanism without their
+    shift: the range in which products of exponentials are used is then that of the others."""
+    import copy
+    mech = M.load("drm19")
+    lumped = copy.deepcopy(mech)
+    lumped.reactions.append(M.Reaction("CH4 => CO2", {mech.index("CH4"): 1}, {mech.index("CO2"): 1}, False,
+                                       "elementary", 1e10, 0.0, 2e4))
+    assert set(hipgen._element_shift(lumped)) == {(0.0, 0.0)}
+    for m, below, inside in ((mech, 0.0, True), (mech, 5.0, False), (lumped, 0.0, True), (lumped, 5.0, False)):
+        T = hipgen.shared_range(m)[0] - below
+        worst = 0.0
+        for r in m.reactions:
+            for side in (r.reactants, r.products):
+                g = sum(c * (M.h_RT(m.species[i], T) - M.s_R(m.species[i], T) + d5 / T - d6)
+                        for i, c in side.items() for d5, d6 in [hipgen._element_shift(m)[i]])
+                worst = max(worst, abs(g), abs(r.beta * np.log(T) - r.Ea / M.R_CAL / T))
+        assert (worst <= hipgen.SHARED_LIMIT) == inside
