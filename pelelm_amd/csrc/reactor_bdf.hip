@@ -616,9 +616,25 @@ __device__ __noinline__ int lu_factor(const CM& mat, const double gamma) {
     for (int i = k + 1; i < N1; ++i) {
       const Real lik = A::at(mat, i, k) * inv;
       A::at(mat, i, k) = lik;
-      if (lik != (Real)0) {
+      if (lik != (Real)0) {   // zero in every lane for the Jacobian's structural zeros
+        // four entries at a time, their loads ahead of the stores that might alias them: a
+        // lane's walk along a row of factors stored by columns waits for each of its lines
+        // (one at a time: drm19 20,000 cells 60.8 ms a call against 47.9, 53 species 4,096
+        // cells 1,790 against 1,100)
+        int j = k + 1;
 #pragma unroll 1
-        for (int j = k + 1; j < N1; ++j) A::at(mat, i, j) -= lik * A::at(mat, k, j);
+        for (; j + 4 <= N1; j += 4) {
+          Real u[4], v[4];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            u[t] = A::at(mat, k, j + t);
+            v[t] = A::at(mat, i, j + t);
+          }
+#pragma unroll
+          for (int t = 0; t < 4; ++t) A::at(mat, i, j + t) = v[t] - lik * u[t];
+        }
+#pragma unroll 1
+        for (; j < N1; ++j) A::at(mat, i, j) -= lik * A::at(mat, k, j);
       }
     }
   }
