@@ -4024,17 +4024,23 @@ hipError_t run_trips_graph(const ReactArgs& a, hipStream_t stream, long max_trip
   return hipSuccess;
 }
 
-// Boxes up to batch_cells cells run BATCH_TRIPS trips between two looks at the device's
-// counts, with grids for every cell; above, each trip's grids fit its lists.  A look costs
-// 35 us of idle GPU per trip, a third of a trip on a LiDryer 16^3 box (5.5 -> 4.0 ms per
-// call; drm19 16^3 with GMRES 9.3 -> 8.8, 17x15x13 with forcing 10.6 -> 10.0); a trip after
-// the last cell has finished, 25 us of empty kernels.  The line lies where a factorisation
-// grid's empty blocks cost less than the look: 10 ns a block of one wave (56 species,
-// 29,667 blocks: 0.3 ms a trip, a call 101 -> 157 ms), 46 of two waves (88 species, 32,768
-// blocks: 446 -> 709 ms); two cells share a block up to 32 unknowns.
+// Where trips come in batches: BATCH_TRIPS of them between two looks at the device's counts,
+// with grids for every cell.  A look costs 35 us of idle GPU, unless the trip's evaluation
+// runs beside it (the plain schedule, below); a batch costs the kernels that a look would
+// have left out or made smaller.  Measured, ms per call, one by one / in batches:
+//   GMRES, which has no set-up or factorisation: 9 species plain 4,096 cells 6.14 / 6.02,
+//     32,000 7.12 / 7.04, compacted 7.54 / 6.59 and 9.01 / 8.15; drm19 16,000 cells 20.13 /
+//     20.10 and 23.6 / 22.8: always, as far as that was tried.
+//   compacted lists, direct solve: 9 species 4,096 cells 4.98 / 4.38, 16,000 5.55 / 5.33,
+//     32,000 6.32 / 6.55; drm19 4,096 cells 10.1 / 10.3 (smooth states 5.17 / 5.39): the
+//     smallest mechanisms.
+//   plain schedule, direct solve: 9 species 64 cells 3.50 / 3.52, 4,096 3.97 / 4.01; drm19
+//     300 cells 7.6 / 8.1, 4,096 8.7 / 9.7; 53 species 64 cells 59 / 77, 2,048 83 / 100; 88
+//     species 64 cells 112 / 123: never.
 template <int N1>
-constexpr long batch_cells() {
-  return N1 <= 32 ? 4096 : N1 <= 64 ? 2048 : 512;
+bool in_batches(const ReactArgs& a) {
+  if (a.gmres) return a.ncell <= 32768;
+  return a.compact && N1 <= 16 && a.ncell <= 16384;
 }
 constexpr int BATCH_TRIPS = 8;
 
@@ -4069,9 +4075,9 @@ hipError_t run_react_t(ReactArgs a, hipStream_t stream, long max_trips, long* tr
   int cur = 0;
   long trip = 0;
   unsigned int h_counts[8];
-  // small boxes: several trips per look at the counts (not while profiling, which wants
-  // each launch's cells, nor with the predictor, whose list's count is counts[7])
-  const int batch = (n <= batch_cells<M::N1>() && !prof && !a.use_pred) ? BATCH_TRIPS : 1;
+  // several trips per look at the counts (not while profiling, which wants each launch's
+  // cells, nor with the predictor, whose list's count is counts[7])
+  const int batch = (in_batches<M::N1>(a) && !prof && !a.use_pred) ? BATCH_TRIPS : 1;
   while (batch > 1 && trip < max_trips) {
     const int k = (int)(max_trips - trip < batch ? max_trips - trip : batch);
     for (int t = 0; t < k; ++t) {

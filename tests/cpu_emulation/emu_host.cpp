@@ -56,10 +56,11 @@ thread_local Idx3 threadIdx, blockIdx, blockDim, gridDim;
 using namespace pelelm;
 
 // One react call on flat cell-fastest arrays.  ahead = 1 gives the call the pinned counts
-// and the event with which it issues a trip's evaluation before it waits; out: kernels
+// and the event with which it issues a trip's evaluation before it waits; profile = 1 has
+// its kernels timed, for which trips come one by one and each evaluation after the wait; out: kernels
 // launched, kernels not waited for at the return, looks at the device's counts, trips.
 extern "C" int host_react(long ncell, double* rY, double* T, double* rE, double* FC, double dt, double rtol,
-                          double atol, int compact, int gmres, int ahead, long max_trips, unsigned long long* counters,
+                          double atol, int compact, int gmres, int ahead, int profile, long max_trips, unsigned long long* counters,
                           long* out) {
   const MechTable* t = PELE_TU_MECH_FN();
   const int N = t->nspec;
@@ -100,7 +101,8 @@ extern "C" int host_react(long ncell, double* rY, double* T, double* rE, double*
     plan.counted = &event;
   }
   host::launched = host::waited = host::looks = host::recorded = 0;
-  const int rc = (int)t->run_react(a, nullptr, max_trips, &out[3], nullptr, nullptr, plan);
+  KernelProf prof{};
+  const int rc = (int)t->run_react(a, nullptr, max_trips, &out[3], profile ? &prof : nullptr, nullptr, plan);
   out[0] = host::launched;
   out[1] = host::launched - host::waited;
   out[2] = host::looks;

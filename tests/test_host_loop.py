@@ -4,9 +4,8 @@ The workspace, lists and counts belong to the reactor, and the next call may com
 another stream, which nothing orders behind the first: a kernel of the first call still
 running then would read the second call's cells and append to its lists, beyond their
 ends.  emu_host.cpp counts the launches that the host has waited for, on every way out of
-the loop: trips issued in batches (small boxes) and one by one, the evaluation issued
-before the wait and after it, plain and compacted lists, all cells done and the cap on
-trips reached.
+the loop: trips issued in batches and one by one, the evaluation issued before the wait
+and after it, plain and compacted lists, all cells done and the cap on trips reached.
 """
 import ctypes as C
 import glob
@@ -26,7 +25,7 @@ SRC = [os.path.join(EMU, "emu_host.cpp"), os.path.join(EMU, "hip", "hip_runtime.
 SRC += [os.path.join(CSRC, f) for f in ("reactor_bdf.hip", "reactor_internal.h", "mlp_internal.h")]
 SRC += sorted(glob.glob(os.path.join(CSRC, "mech", "*.inc")))
 CLANG = "/opt/rocm/llvm/bin/clang++"
-MECH, LIMIT = "LiDryer", 4096   # the most cells of a box of this mechanism whose trips come in batches
+MECH, N = "LiDryer", 1000
 
 
 @pytest.fixture(scope="module")
@@ -40,27 +39,27 @@ def lib():
     return C.CDLL(out)
 
 
-def _react(lib, d, n, compact, gmres, ahead, cap):
+def _react(lib, d, n, compact, gmres, ahead, cap, profile=0):
     p = lambda a: a.ctypes.data_as(C.c_void_p)  # noqa: E731
     rY, T, rE = (d[k][..., :n].copy() for k in ("rY", "T", "rE"))
     FC, cnt, out = np.zeros(n), np.zeros(16, dtype=np.uint64), (C.c_long * 4)()
     rc = lib.host_react(C.c_long(n), p(rY), p(T), p(rE), p(FC), C.c_double(d["dt"]), C.c_double(1e-6),
-                        C.c_double(1e-10), compact, gmres, ahead, C.c_long(cap), p(cnt), out)
+                        C.c_double(1e-10), compact, gmres, ahead, profile, C.c_long(cap), p(cnt), out)
     assert rc == 0
     return rY, T, FC, cnt, {"launched": out[0], "left": out[1], "looks": out[2], "trips": out[3]}
 
 
 @pytest.fixture(scope="module")
 def box():
-    return cells.generate_workload("lidryer_16", ncell=LIMIT + 1)
+    return cells.generate_workload("lidryer_16", ncell=N)
 
 
-@pytest.mark.parametrize("n", [130, LIMIT + 1])
+@pytest.mark.parametrize("n", [130, N])
 @pytest.mark.parametrize("compact,gmres", [(0, 0), (1, 0), (0, 1)])
-@pytest.mark.parametrize("ahead", [0, 1])
+@pytest.mark.parametrize("ahead,profile", [(0, 0), (1, 0), (1, 1)])
 @pytest.mark.parametrize("cap", [60100, 19])
-def test_no_kernel_outlives_the_call(lib, box, n, compact, gmres, ahead, cap):
-    FC, cnt, out = _react(lib, box, n, compact, gmres, ahead, cap)[2:]
+def test_no_kernel_outlives_the_call(lib, box, n, compact, gmres, ahead, profile, cap):
+    FC, cnt, out = _react(lib, box, n, compact, gmres, ahead, cap, profile)[2:]
     assert out["launched"] > 0
     assert out["left"] == 0
     if cap == 19:   # no multiple of a batch: exactly 19 trips, and every unfinished cell failed
@@ -72,16 +71,15 @@ def test_no_kernel_outlives_the_call(lib, box, n, compact, gmres, ahead, cap):
 @pytest.mark.parametrize("compact,gmres", [(0, 0), (1, 0), (0, 1), (1, 1)])
 @pytest.mark.parametrize("cap", [60100, 19])
 def test_batches_and_early_evaluations_change_nothing(lib, box, compact, gmres, cap):
-    """The same cells with their trips in batches of eight, one by one, and one by one with
-    the evaluation issued before the wait: the same states, counts and number of trips."""
-    runs = [_react(lib, box, LIMIT, compact, gmres, 0, cap)] + \
-        [_react(lib, box, LIMIT + 1, compact, gmres, ahead, cap) for ahead in (0, 1)]
-    batched, single, early = runs
-    for other in (single, early):
-        for a, b in zip(batched[:3], other[:3]):
-            np.testing.assert_array_equal(a[..., :LIMIT], b[..., :LIMIT])
-        assert batched[4]["trips"] == other[4]["trips"]
-    trips = batched[4]["trips"]
-    assert batched[4]["looks"] == -(-trips // 8)
-    assert single[4]["looks"] == early[4]["looks"] == trips + (cap != 19)
-    np.testing.assert_array_equal(single[3], early[3])
+    """The same cells with their trips as the call issues them (in batches of eight for
+    compacted lists and GMRES, else each evaluation before the wait), without the early
+    evaluation, and one by one: the same states, counts and number of trips."""
+    usual, late, single = [_react(lib, box, N, compact, gmres, ahead, cap, profile)
+                           for ahead, profile in ((1, 0), (0, 0), (1, 1))]
+    for other in (late, single):
+        for a, b in zip(usual[:4], other[:4]):
+            np.testing.assert_array_equal(a, b)
+        assert usual[4]["trips"] == other[4]["trips"]
+    trips = usual[4]["trips"]
+    assert single[4]["looks"] == trips + (cap != 19)
+    assert usual[4]["looks"] == (-(-trips // 8) if compact or gmres else trips + (cap != 19))
