@@ -80,14 +80,14 @@ def mech_ops(mech: str):
 
 
 def rhs_ops(mech: str):
-    """Algorithmic flops of one right-hand-side evaluation (fixed part, per HY2T
-    iteration) and its transcendentals, from the generator's static counts."""
+    """Flops of one right-hand-side evaluation as the kernels do it (fixed part, per HY2T
+    iteration) and its transcendentals, from the generator's counts of the emitted code."""
     ops = mech_ops(mech)
-    d, N = ops["functions"], ops["nspec"]
-    cph = d["thermo_cph"]["flops"]
-    # rho, 1/rho, Y; after HY2T: log T, 1/T, C, gibbs, wdot, cp/h, f, rho cp, h.wdot, fT
-    fixed = (2 * N + 1) + 2 + N + d["gibbs"]["flops"] + d["wdot"]["flops"] + cph + 7 * N + 5
-    per_iter = cph + 6 * N + 5
+    d, N = ops["emitted"], ops["nspec"]
+    # the mixture's coefficients (HY2T starts with them) and cp, log T, 1/T, C, gibbs, wdot,
+    # f, and the enthalpy of f's mixture for dT/dt
+    fixed = d["mix"]["flops"] + 9 + 1 + N + d["gibbs"]["flops"] + d["wdot"]["flops"] + 2 * N + d["mix"]["flops"] + 18
+    per_iter = 15 + 8 + 5   # the two polynomials h and cp of the mixture, and the step
     trans = 1 + d["wdot"]["transcendentals"]
     return fixed, per_iter, trans
 
@@ -99,13 +99,15 @@ def bytes_per_cell(nspec: int) -> int:
 
 
 LANE_WORDS = 53   # 8-byte words of the integrator's stored lane state (independent of the mechanism)
+EVAL_LANE_WORDS = 10   # the words of it that k_eval reads
 
 
 def rhs_bytes(N: int) -> int:
-    """Workspace bytes one k_eval cell-evaluation moves: zn0, zn1, acor, forcing and the
-    lane state read, y, f and T written."""
+    """Workspace bytes one k_eval cell-evaluation of a Newton iteration moves: zn0, zn1, acor,
+    the forcing and the lane state's words it uses read, the Newton system's right-hand side
+    written (y, f and T only where a set-up or a start-up phase follows)."""
     N1 = N + 1
-    return 8 * (3 * N1 + N + LANE_WORDS + 2 * N1 + 1)
+    return 8 * (3 * N1 + N + EVAL_LANE_WORDS + N1)
 
 
 KINDS = ["k_eval", "k_setup", "k_consume", "k_lu_coop", "k_predict", "k_solve_coop"]
@@ -116,12 +118,12 @@ KIND_DESC = {"k_eval": "right-hand side (HY2T, rates, energy)", "k_setup": "anal
 
 
 def kernel_model(st, nspec, mech):
-    """Algorithmic work of each kernel kind over the call: (FP64 flops, workspace bytes).
+    """Work of each kernel kind over the call: (FP64 flops, workspace bytes).
     The Newton update and step logic count 8 n per iteration (update, WRMS norm) and
     2 * 5n * 3 per step (Nordsieck predict, correct, error weights)."""
     N, n = nspec, nspec + 1
     fixed, per_iter, _ = rhs_ops(mech)
-    jac_flops = mech_ops(mech)["functions"]["jacobian"]["flops"]
+    jac_flops = mech_ops(mech)["emitted"]["jacobian"]["flops"]
     nfe, nni, nst, nsetups, nje = st["nfe"], st["nni"], st["nsteps"], st["nsetups"], st["nje"]
     evals = st["kernel_cells"][0] or nfe
     consume_passes = st["kernel_cells"][2] or nfe

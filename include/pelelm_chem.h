@@ -7,8 +7,9 @@
  * the absolute tolerances, asked to react boxes, closed at teardown.  Every entry point
  * takes plain pointers and sizes; device arrays are HIP device pointers and all work is
  * enqueued on the caller's HIP stream.  The host-driven schedules (plain, queue, auto)
- * read the work-list counts back once per trip (small boxes once per eight trips, captured
- * graphs once per graph), and react returns with every kernel of the integration finished
+ * read the work-list counts back once per trip (GMRES boxes up to 32,768 cells, and
+ * compacted lists of the smallest mechanisms, once per eight trips; captured graphs once per
+ * graph), and react returns with every kernel of the integration finished
  * (the reference's caller synchronises right after the call anyway,
  * Source/PeleLM.cpp:5773-5775), so the next call may use another stream; the persistent
  * schedule and ReactorRK64 enqueue one kernel and synchronise only to read the failure
@@ -140,7 +141,8 @@ int mi_chem_init(void* reactor, int reactor_type, int ncells);
      cvode.max_num_steps + 100; cells still integrating after this many trips fail),
      mi.on_fail (abort: react returns MI_ECELLFAIL when a cell failed, default | continue:
      react returns MI_OK, failed cells carry FC < 0), mi.profile (0 | 1: per-kernel event
-     timing). */
+     timing; trips are then issued one by one, each after the counts of the one before, so a
+     small box takes longer than it does unprofiled). */
 int mi_chem_set(void* reactor, const char* key, const char* value);
 
 /* ReactorBase::set_typ_vals_ode -- Source/PeleLM.cpp:1497-1516: n = nspec + 1 typical

@@ -2009,7 +2009,10 @@ __device__ __forceinline__ int lu_coop_core(const CM& mat, const bool work, cons
       // one cell per wave, FP64: the pivot row's entries are read from lane `who`
       // (uniform) with v_readlane.  The multiplier is zero in the lanes whose row stays as
       // it is, so the updates need no mask (which the compiler makes two selects per
-      // entry).  (The FP32 factorisation measured faster with the LDS broadcast below.)
+      // entry).  Only a pivot row with an infinity or a NaN reaches rows that a mask would
+      // have kept, as 0 x inf; every solution by such factors is NaN either way, and the
+      // Newton iteration rejects it.  (The FP32 factorisation measured faster with the LDS
+      // broadcast below, where a zero multiplier does leave its row.)
       const Real pk = lane_read(m[k], who), pb = lane_read(bv, who);
       const Real l = upd ? m[k] * ((Real)1 / pk) : (Real)0;
       if (upd) m[k] = l;

@@ -29,8 +29,9 @@ T* = 1e30 vanish / become constants; third-body sums start from the total concen
 and add (eff - 1) C_k only for species with non-unit efficiency.
 
 ``gen_thermo``, ``gen_wdot`` and ``gen_jacobian(shared=False)`` write the same arithmetic
-out species by species and reaction by reaction; the operation counts are counted on that
-form, which says what a mechanism asks for and not how the emitted code saves on it.
+out species by species and reaction by reaction; the operation counts "functions" are
+counted on that form, which says what a mechanism asks for and not how the emitted code
+saves on it, and "emitted" on the code that runs.
 """
 from __future__ import annotations
 
@@ -767,6 +768,27 @@ def count_ops(code: str) -> dict:
     return {"flops": flops, "transcendentals": sum(trans.values()), "by_function": trans}
 
 
+def emitted_counts(mech: M.Mechanism) -> dict:
+    """Operation counts of the emitted code, for one side of the fits' break temperature:
+    ``mix`` (the mixture's coefficients), ``gibbs``, ``wdot`` and ``jacobian``."""
+    ns = mech.nspec
+    loops = re.compile(r"k < NS; \+\+k\) \{ (.*) \}$")
+
+    def flat(code):   # loops over the species as count_ops knows them, a statement a line
+        out = []
+        for line in code.splitlines():
+            m = loops.search(line)
+            out += [f"for (int k = 0; k < {ns}; ++k) {t};" for t in m.group(1).split("; ")] if m else \
+                [line.replace("k < NS;", f"k < {ns};")]
+        return "\n".join(out)
+
+    thermo = {}
+    for part in gen_thermo(mech).split("static __device__ __forceinline__ void ")[1:]:
+        thermo[part.split("(")[0]] = count_ops(part)
+    return {"mix": {"flops": 12 * ns, "transcendentals": 0}, "gibbs": thermo["gibbs"],
+            "wdot": count_ops(flat(gen_wdot_shared(mech))), "jacobian": count_ops(flat(gen_jacobian(mech)))}
+
+
 def write_inc(mech: M.Mechanism, path: str) -> None:
     ns = mech.nspec
     name = mech.name
@@ -799,12 +821,6 @@ def write_inc(mech: M.Mechanism, path: str) -> None:
         counts[fname] = count_ops(part)
     counts["wdot"] = count_ops(wd)
     counts["jacobian"] = count_ops(jac)
-    lines.append("// static operation counts (flops; transcendentals) of the functions, written out species by")
-    lines.append("// species and reaction by reaction")
-    for k, v in counts.items():
-        lines.append(f"static constexpr long OPS_{k.upper()} = {v['flops']};")
-        lines.append(f"static constexpr long TRANS_{k.upper()} = {v['transcendentals']};")
-    lines.append("")
     lines.append(gen_thermo_tables(mech))
     lines.append("")
     lines.append(gen_wdot_shared(mech))
@@ -818,4 +834,7 @@ def write_inc(mech: M.Mechanism, path: str) -> None:
         f.write("\n".join(lines) + "\n")
     ops_path = os.path.join(os.path.dirname(os.path.dirname(path)), "..", "mechanisms", f"{name}_ops.json")
     with open(os.path.normpath(ops_path), "w") as f:
-        json.dump({"mechanism": name, "nspec": ns, "nreac": mech.nreac, "functions": counts}, f, indent=1)
+        # "functions": written out species by species and reaction by reaction, what the model
+        # asks for; "emitted": the code that runs, one range of the NASA fits
+        json.dump({"mechanism": name, "nspec": ns, "nreac": mech.nreac, "functions": counts,
+                   "emitted": emitted_counts(mech)}, f, indent=1)
